@@ -726,7 +726,7 @@ int v7g_swiglu_f32(float *out, const float *gate, const float *up, long long n) 
 static int check_quant(const int8_t *out_q, const float *out_s, int rows, int row_len, int gs) {
   if (rows < 0 || row_len <= 0 || gs < 1 || gs > 4096) return V7G_ERR_SHAPE;
   if ((long long)rows * row_len >= (1LL << 40)) return V7G_ERR_SHAPE;
-  // the general path runs one thread per group in 256-thread blocks: at most 2^30 blocks
+  // groups stay countable in 64-bit lane indices (at most 64 lanes each)
   if ((long long)rows * ((row_len + gs - 1) / gs) >= (1LL << 38)) return V7G_ERR_SHAPE;
   if (rows == 0) return V7G_OK;
   if (!out_q || !out_s) return V7G_ERR_NULL;

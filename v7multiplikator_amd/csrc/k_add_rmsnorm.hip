@@ -15,8 +15,13 @@
 // residual and add together and pass 2 needs no second read; residual, add
 // and o move as streaming loads and stores, the weight row stays cached.  The
 // updated residual also goes to LDS, where 32 lanes of wave 0 replay the 32
-// FMA chains (lane 8q + j is accumulator q, YMM lane j), conflict-free; the
-// five-step xor exchange below is exactly the (A+B)+(C+D) + HADD_YMM pairing.
+// FMA chains, chain by chain (ChainLayout), and reduce them with DPP row
+// shifts in the (A+B)+(C+D) + HADD_YMM pairing.
+// Bound: many rows by HBM ([8192, 4096] add+RMSNorm 85-86 us, 79% of the peak;
+// [1000, 16384] 53.2 -> 46.2 us with 1024 threads per row in place of 256); few
+// rows by latency: the loads, the chain (128 dependent FMAs at 4096 floats),
+// the scale's divisions and square root, the stores ([8, 4096] RMSNorm 3.29 ->
+// 2.67 us, add+RMSNorm -> Q8 3.49 -> 3.36, [8, 5376] add+RMSNorm 5.4 -> 3.4).
 //
 // The same row body serves the neighbours of this kernel in the reference:
 //   v7s_rmsnorm (src/asm/rmsnorm_kernel.inc:12-75): no add, same order;
@@ -45,6 +50,18 @@ __device__ __forceinline__ int chain_of_lane(int lam) {
 template <int CTRL>
 __device__ __forceinline__ float dpp_f(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
+
+// The reference's reduction of the 32 chains (lane lam holds chain
+// chain_of_lane(lam)) as DPP row shifts; the same value in every lane.
+__device__ __forceinline__ float chain_reduce(float acc) {
+  acc = acc + dpp_f<0x108>(acc);  // row_shl:8   A+B, C+D
+  acc = acc + dpp_f<0x104>(acc);  // row_shl:4   (A+B)+(C+D)
+  acc = acc + dpp_f<0x102>(acc);  // row_shl:2   HADD_YMM: v_i + v_{i+4}
+  acc = acc + dpp_f<0x101>(acc);  // row_shl:1   w0+w1, w2+w3
+  const float lo = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, acc), 0));
+  const float hi = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, acc), 16));
+  return lo + hi;
 }
 
 // Sum of squares of a row of dim floats (dim % 32 == 0) staged at the padded
@@ -97,13 +114,7 @@ __device__ __forceinline__ float padded_row_sumsq(const float *row, int dim) {
       }
     }
   }
-  acc = acc + dpp_f<0x108>(acc);  // row_shl:8   A+B, C+D
-  acc = acc + dpp_f<0x104>(acc);  // row_shl:4   (A+B)+(C+D)
-  acc = acc + dpp_f<0x102>(acc);  // row_shl:2   HADD_YMM: v_i + v_{i+4}
-  acc = acc + dpp_f<0x101>(acc);  // row_shl:1   w0+w1, w2+w3
-  const float lo = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, acc), 0));
-  const float hi = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, acc), 16));
-  return lo + hi;
+  return chain_reduce(acc);
 }
 
 // A workgroup barrier for LDS only: unlike __syncthreads() it does not wait
@@ -112,118 +123,197 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 
 __device__ __forceinline__ int padded(int m) { return 4 * (m + (m >> 2)); }
 
-// One row.  ADD: the input is residual + add (residual updated in place),
-// else x.  QGS == 0: o = (s*x)*w; QGS = 32 or 64: the normalised row is
-// quantized in groups of QGS (codes q, scales q_s) and o is not written.
-// o may alias residual (the row then ends as o, as in the reference).
-// PAD (dim % 32 == 0, dim <= 12288): the row is staged at the padded layout and
-// the chains' reduction runs as DPP row shifts (padded_row_sumsq); otherwise
-// at the natural layout with the lane-exchange reduction, which also covers
-// the leftover 8-float blocks of dim % 32 != 0.
-// FIX (with PAD, dim == 4*TPR*KMAX): every chunk is live, so the loads and
-// stores carry no bounds branches (whose merges cost waits on the outstanding
-// loads); the fused-add form then also requests its weights right after the
-// row's loads, ahead of the residual's stores, since vector memory operations
-// retire in issue order and a weight load issued after those stores would
-// wait for them (KMAX <= 4: with more chunks the weights would not fit in 64
-// VGPRs beside the row).  TPR == 0 (FIX only): the thread count is the
-// launch's blockDim.x and dim = 4*blockDim.x*KMAX; a compile-time TPR folds
-// the chunk offsets into the instructions and measured about 2% faster.
-template <int TPR, int KMAX, bool ADD, int QGS, bool PAD, bool FIX = false>
+// Where the row kernels stage a row: chain by chain.  Chain lane lam's
+// elements, in the order its FMAs take them, lie one behind another at float
+// lam * STRIDE, so the lane reads four of them with one 16-byte LDS load.
+// Element 8b + j of the row (block b, YMM lane j) is step left + g of its chain
+// for block left + 4g + q; the leftover blocks b < left = (dim/8) % 4, which
+// the reference takes first, all into A, are steps b of chain (A, j).  Steps a
+// chain has no element for (past the row's end; B, C and D during the leftover
+// blocks) hold zeros: fma(0, 0, acc) is acc for every sum of squares, so they
+// change nothing, and every row of up to 4*TPR*KMAX floats runs the same
+// compiled chain.
+// U: 16-byte reads per register set of the chain.
+template <int TPR, int KMAX, bool LEFT, int U>
+struct ChainLayout {
+  static constexpr int kSteps = TPR * KMAX / 8 + (LEFT ? 3 : 0);  // room for three leftover blocks
+  static constexpr int kSets = (kSteps + 4 * U - 1) / (4 * U);
+  static constexpr int kStride = 4 * U * kSets + 4 * (1 + (U * kSets) % 2);
+  static_assert(kStride % 8 == 4, "the 16-byte reads of 16 lanes, and a wave's 4-byte writes, fall on distinct banks");
+  // two sets behind the last chain, which the chain's prefetch touches; then the scale
+  static constexpr int kScale = 32 * kStride + 8 * U;
+  static constexpr unsigned kBytes = 4u * (kScale + 4);
+};
+
+// The row's sum of squares in the reference's order, from the chain layout;
+// called by a whole wave, the same value in every lane.  Three register sets of
+// U 16-byte reads: two sets are in flight while the FMAs consume the third (LDS
+// answers in about 130 cycles, a set of U = 4 is 16 dependent FMAs of 4 cycles).
+// The empty asm statements pass the accumulator through a point after each set
+// of reads, so the compiler neither sinks a read to its use nor hoists the FMAs
+// above the reads of another set.  Reads run up to two sets past the chain's
+// end, into the next chain or the space behind the last.
+template <int SETS, int STRIDE, int U>
+__device__ __forceinline__ float chain_sumsq(const float *row) {
+  const int lane = __lane_id();
+  float acc = 0.0f;
+  if (lane < 32) {
+    const float4 *p = reinterpret_cast<const float4 *>(row + lane * STRIDE);
+    float4 a[U], b[U], d[U];
+    auto get = [&](float4(&v)[U], int set) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = p[U * set + u];
+      asm volatile("" : "+v"(acc)::"memory");
+    };
+    auto eat = [&](const float4(&v)[U]) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        acc = __builtin_fmaf(v[u].x, v[u].x, acc);
+        acc = __builtin_fmaf(v[u].y, v[u].y, acc);
+        acc = __builtin_fmaf(v[u].z, v[u].z, acc);
+        acc = __builtin_fmaf(v[u].w, v[u].w, acc);
+      }
+      asm volatile("" : "+v"(acc)::"memory");
+    };
+    get(a, 0);
+    get(b, 1);
+    for (int s = 0;; s += 3) {
+      get(d, s + 2);
+      eat(a);
+      if (s + 1 >= SETS) break;
+      get(a, s + 3);
+      eat(b);
+      if (s + 2 >= SETS) break;
+      get(b, s + 4);
+      eat(d);
+      if (s + 3 >= SETS) break;
+    }
+  }
+  return chain_reduce(acc);
+}
+
+// One row of dim floats, 4*TPR*(KMAX-1) < dim <= 4*TPR*KMAX.  ADD: the input
+// is residual + add (residual updated in place), else x.  QGS == 0:
+// o = (s*x)*w; QGS = 32 or 64: the normalised row is quantized in groups of
+// QGS (codes q, scales q_s) and o is not written.  o may alias residual (the
+// row then ends as o, as in the reference).  LEFT: dim % 32 != 0.
+// Each of TPR threads holds KMAX float4 chunks in registers from the loads to
+// the results.  Only the last chunk is tested against the row's end: its loads
+// are clamped to the row's first floats, its LDS stores are zeros, its global
+// stores predicated (a branch around a load would put a wait at its merge).
+// When the weights are requested (vector memory operations retire in issue
+// order, so a weight load behind the residual's stores waits for them):
+//  - FEW, at most one row per CU: once the row is staged, ahead of the
+//    residual's stores, so that they travel during the chain and delay neither
+//    the row nor the result ([1, 8192] add+RMSNorm 4.85 -> 4.02 us, with the
+//    chain's new layout);
+//  - many rows, ADD: right behind the row's loads;
+//  - many rows without ADD: after the chain, so that the other rows on the CU
+//    get their loads first ([1024, 4096] 6.9 -> 6.2 us); with four and more
+//    chunks one by one, each store waiting for the one before (and so with ADD
+//    beyond 8192 floats at two rows per CU).  Where all rows are resident at
+//    once, unpaced stores of the first rows hold up the loads of the last: [1000,
+//    8192] 14.4 us, paced 11.4.
+// FEW uses as many registers as the chain can use; otherwise at most 64 VGPRs
+// (row_waves), so that a CU's waves are full, with smaller chain sets.
+static constexpr int row_chain_u(int kmax, bool few) { return few || kmax == 1 ? 4 : (kmax == 2 ? 3 : 2); }
+
+template <int TPR, int KMAX, bool ADD, int QGS, bool LEFT, bool FEW>
 __device__ __forceinline__ void rms_row(float *o, int8_t *q, float *q_s, float *xin, const float *add,
                                         const float *weight, int dim, float eps) {
-  static_assert(!FIX || PAD, "the fixed-length row uses the padded layout");
-  static_assert(TPR > 0 || (FIX && QGS == 0), "a run-time thread count only for the fixed-length row");
-  constexpr bool EARLY_W = FIX && ADD && QGS == 0 && KMAX <= 4;
-  const int tpr = TPR ? TPR : (int)blockDim.x;
-  if constexpr (FIX) dim = 4 * tpr * KMAX;
+  constexpr int U = row_chain_u(KMAX, FEW);
+  using L = ChainLayout<TPR, KMAX, LEFT, U>;
+  constexpr int STRIDE = L::kStride;
+  constexpr bool LATE_W = !FEW && (!ADD || (KMAX == 8 && TPR > 256));
   extern __shared__ __attribute__((aligned(16))) float row[];
   const int tid = threadIdx.x;
   const size_t r = blockIdx.x;
   float *xr = xin + r * (size_t)dim;
+  const float *ar = ADD ? add + r * (size_t)dim : nullptr;
+  const bool last = 4 * (tid + (KMAX - 1) * TPR) < dim;  // the last chunk is live
+  auto live = [&](int k) { return LEFT ? 4 * (tid + k * TPR) < dim : k < KMAX - 1 || last; };
+  // A chunk's address as a uniform base and a 32-bit lane offset (scalar-base loads and stores).
+  const unsigned t4 = 4u * (unsigned)tid;
+  const unsigned t4_last = last ? t4 + 4u * (KMAX - 1) * TPR : 0u;
+  auto src = [&](const float *p, int k) {
+    if constexpr (LEFT) return p + (live(k) ? t4 + 4u * k * TPR : 0u);
+    return k < KMAX - 1 ? (p + 4 * k * TPR) + t4 : p + t4_last;
+  };
 
-  // Pass 1: load the row (and add), stage it in LDS.
-  float4 x[KMAX], b[KMAX], w_early[EARLY_W ? KMAX : 1];
+  float4 x[KMAX], b[KMAX], w[KMAX];
 #pragma unroll
   for (int k = 0; k < KMAX; ++k) {
-    const int i = 4 * (tid + k * tpr);
-    if (FIX || i < dim) {
-      x[k] = ld_stream4(xr + i);
-      if constexpr (ADD) b[k] = ld_stream4(add + r * (size_t)dim + i);
-    }
+    x[k] = ld_stream4(src(xr, k));
+    if constexpr (ADD) b[k] = ld_stream4(src(ar, k));
   }
-  if constexpr (EARLY_W) {
+  auto load_w = [&]() {
 #pragma unroll
-    for (int k = 0; k < KMAX; ++k) w_early[k] = *reinterpret_cast<const float4 *>(weight + 4 * (tid + k * tpr));
-  }
-#pragma unroll
-  for (int k = 0; k < KMAX; ++k) {
-    const int i = 4 * (tid + k * tpr);
-    if (FIX || i < dim) {
-      if constexpr (ADD) {
-        x[k] = make_float4(x[k].x + b[k].x, x[k].y + b[k].y, x[k].z + b[k].z, x[k].w + b[k].w);
-        st_stream4(xr + i, x[k]);
-      }
-      *reinterpret_cast<float4 *>(row + (PAD ? padded(tid + k * tpr) : i)) = x[k];
+    for (int k = 0; k < KMAX; ++k) w[k] = *reinterpret_cast<const float4 *>(src(weight, k));
+  };
+  if constexpr (ADD && !FEW && !LATE_W) load_w();
+  const int left = LEFT ? (dim >> 3) & 3 : 0;
+  {  // zeros for the steps no chunk writes
+    constexpr int first = LEFT ? 0 : TPR * KMAX / 8, end = 4 * U * L::kSets;
+    for (int i = tid + 32 * first; i < 32 * end; i += TPR) {
+      const int lam = i & 31, step = i >> 5;
+      const bool zero = !LEFT || (step < left && chain_of_lane(lam) >= 8) || step >= left + (dim >> 5);
+      if (zero) row[lam * STRIDE + step] = 0.f;
     }
   }
-  __syncthreads();
-
-  if constexpr (PAD) {
-    // floats 16..19 of the padded layout are padding: the scale goes there
-    if (tid < 64) {
-      const float s0 = rms_scale(padded_row_sumsq<8>(row, dim), (float)dim, eps);
-      if (tid == 0) row[16] = s0;
-    }
-  } else if (tid < 64) {
-    // The 32 FMA chains: lane v = 8q + j is YMM accumulator q (A..D), lane j.
-    float acc = 0.0f;
-    if (tid < 32) {
-      const int qa = tid >> 3, j = tid & 7;
-      const int blocks = dim >> 3, left = blocks & 3, groups = blocks >> 2;
-      if (qa == 0)
-        for (int bb = 0; bb < left; ++bb) {
-          const float v = row[8 * bb + j];
-          acc = __builtin_fmaf(v, v, acc);
-        }
-      const float *p = row + 8 * (left + qa) + j;
-#pragma unroll 16
-      for (int g = 0; g < groups; ++g) {
-        const float v = p[32 * g];
-        acc = __builtin_fmaf(v, v, acc);
-      }
-    }
-    // (A+B), (C+D): xor 8; then their sum: xor 16; HADD_YMM: xor 4, xor 1, xor 2.
-    acc = acc + xor_f(acc, 8);
-    acc = acc + xor_f(acc, 16);
-    acc = acc + xor_f(acc, 4);
-    acc = acc + xor_f(acc, 1);
-    acc = acc + xor_f(acc, 2);
-    // row[0] is dead now: only lane 0 read it (its first chain element), and
-    // lane 0 is the writer; the other waves wait at the barrier below.
-    if (tid == 0) row[0] = rms_scale(acc, (float)dim, eps);
-  }
-  __syncthreads();
-  const float s = row[PAD ? 16 : 0];
-
-  // Pass 2: n = (s * x) * w, then either stored or quantized.
 #pragma unroll
   for (int k = 0; k < KMAX; ++k) {
-    const int i = 4 * (tid + k * tpr);
-    const bool live = FIX || i < dim;
-    float4 n = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (live) {
-      float4 w;
-      if constexpr (EARLY_W)
-        w = w_early[k];
-      else
-        w = *reinterpret_cast<const float4 *>(weight + i);
-      n = make_float4((s * x[k].x) * w.x, (s * x[k].y) * w.y, (s * x[k].z) * w.z, (s * x[k].w) * w.w);
+    if constexpr (ADD) x[k] = make_float4(x[k].x + b[k].x, x[k].y + b[k].y, x[k].z + b[k].z, x[k].w + b[k].w);
+    // chunk m is the half (m & 1) of block m >> 1: chains 8q + 4(m & 1) + {0, 1, 2, 3}, which
+    // chain_of_lane gives to lanes lam + {0, 1, 16, 17}
+    const int m = tid + k * TPR, blk = m >> 1;
+    int qa = blk & 3, step = blk >> 2;
+    if constexpr (LEFT) {
+      const bool lo = blk < left;
+      qa = lo ? 0 : (blk - left) & 3;
+      step = lo ? blk : left + ((blk - left) >> 2);
     }
+    float *p = row + (8 * (qa & 1) + 4 * (qa >> 1) + 2 * (m & 1)) * STRIDE + step;
+    if (!LEFT || live(k)) {
+      p[0] = live(k) ? x[k].x : 0.f;
+      p[STRIDE] = live(k) ? x[k].y : 0.f;
+      p[16 * STRIDE] = live(k) ? x[k].z : 0.f;
+      p[17 * STRIDE] = live(k) ? x[k].w : 0.f;
+    }
+  }
+  if constexpr (ADD) {
+    if constexpr (FEW) {
+      asm volatile("" ::: "memory");
+      load_w();
+      asm volatile("" ::: "memory");
+    }
+#pragma unroll
+    for (int k = 0; k < KMAX; ++k)
+      if (live(k)) st_stream4((xr + 4 * k * TPR) + t4, x[k]);
+  }
+  lds_barrier();
+  if constexpr (!ADD && FEW) load_w();
+  if (tid < 64) {
+    const float s0 = rms_scale(chain_sumsq<L::kSets, STRIDE, U>(row), (float)dim, eps);
+    if (tid == 0) row[L::kScale] = s0;
+  }
+  lds_barrier();
+  if constexpr (LATE_W && KMAX < 4) load_w();
+  const float s = row[L::kScale];
+
+  // n = (s * x) * w, then either stored or quantized.
+#pragma unroll
+  for (int k = 0; k < KMAX; ++k) {
+    const unsigned i = 4u * (unsigned)(tid + k * TPR);
+    if constexpr (LATE_W && KMAX >= 4) {  // one chunk's weights, and the stores so far done, before its store
+      w[k] = *reinterpret_cast<const float4 *>(src(weight, k));
+      asm volatile("s_waitcnt vmcnt(0)" : "+v"(w[k].x), "+v"(w[k].y), "+v"(w[k].z), "+v"(w[k].w)::"memory");
+    }
+    const float4 n =
+        make_float4((s * x[k].x) * w[k].x, (s * x[k].y) * w[k].y, (s * x[k].z) * w[k].z, (s * x[k].w) * w[k].w);
     if constexpr (QGS == 0) {
-      if (live) st_stream4(o + r * (size_t)dim + i, n);
+      if (live(k)) st_stream4((o + r * (size_t)dim + 4 * k * TPR) + t4, n);
     } else {
-      // QGS/4 consecutive lanes hold one group (dim % QGS == 0 and TPR % 16 == 0:
+      // QGS/4 consecutive lanes hold one group (dim % QGS == 0 and whole waves:
       // a group is entirely live or entirely past the row); every lane takes
       // part in the DPP butterfly, or, in a wave holding a NaN or an Inf, in
       // the reference's ordered vmaxps tree (rmsnorm_quantize_kernel.inc:158-186).
@@ -239,9 +329,9 @@ __device__ __forceinline__ void rms_row(float *o, int8_t *q, float *q_s, float *
         q8_scale(q8_floor(group_absmax_tree<QGS>(n)), scale, recip);
         codes = pack4_codes_full(n, recip);
       }
-      if (live) {
-        const size_t c = (r * (size_t)dim + i) >> 2;  // dword of 4 codes
-        st_stream_u32(reinterpret_cast<uint32_t *>(q) + c, codes);
+      if (live(k)) {
+        const size_t cw = (r * (size_t)dim + i) >> 2;  // dword of 4 codes
+        st_stream_u32(reinterpret_cast<uint32_t *>(q) + cw, codes);
         if ((tid & (LPG - 1)) == 0) st_stream_f32(q_s + r * (size_t)(dim / QGS) + (i / QGS), scale);
       }
     }
@@ -353,189 +443,234 @@ __global__ __launch_bounds__(TPB ? TPB : 1024) void norm_q8_row16_kernel(int8_t 
   st_stream_f32(q_s + r * (size_t)(dim / QGS) + t / (QGS / 16), scale);
 }
 
-template <int TPR, int KMAX, bool PAD, bool FIX>
-__global__ __launch_bounds__(TPR ? TPR : 1024, (TPR == 0 && KMAX <= 4) ? 8 : 1) void fused_add_rmsnorm_kernel(float *o, float *residual, const float *add,
+// Waves per SIMD: full CUs for many rows; 8 chunks of residual, add and weights need 128 VGPRs.
+static constexpr int row_waves(int kmax, bool add, bool few) { return few ? 1 : (kmax == 8 && add ? 4 : 8); }
+
+template <int TPR, int KMAX, bool ADD, bool LEFT, bool FEW>
+__global__ __launch_bounds__(TPR, row_waves(KMAX, ADD, FEW)) void rmsnorm_row_kernel(float *o, float *x, const float *add,
+                                                                       const float *weight, int dim, float eps) {
+  rms_row<TPR, KMAX, ADD, 0, LEFT, FEW>(o, nullptr, nullptr, x, add, weight, dim, eps);
+}
+
+template <int TPR, int KMAX, int QGS, bool ADD, bool FEW>
+__global__ __launch_bounds__(TPR, FEW ? 1 : 8) void rmsnorm_q8_row_kernel(int8_t *q, float *q_s, float *x,
+                                                                          const float *add, const float *weight,
+                                                                          int dim, float eps) {
+  rms_row<TPR, KMAX, ADD, QGS, false, FEW>(nullptr, q, q_s, x, add, weight, dim, eps);
+}
+
+// Many rows of exactly 4*TPR*KMAX floats with TPR = 256 (1024, 2048, 3072 and
+// 4096): the row staged at the padded layout with one 16-byte LDS store per
+// chunk, which costs the other rows on the CU less than rms_row's four 4-byte
+// ones; their waves hide the longer chain.  [8192, 4096] add+RMSNorm: 86.3 us
+// against rms_row's 89.2; [2048, 2048] 13.1 against 12.7, [512, 2048] 3.95
+// against 4.35.
+template <int KMAX, bool ADD>
+__global__ __launch_bounds__(256) void rmsnorm_fixed_row_kernel(float *o, float *xin, const float *add,
                                                                 const float *weight, int dim, float eps) {
-  rms_row<TPR, KMAX, true, 0, PAD, FIX>(o, nullptr, nullptr, residual, add, weight, dim, eps);
-}
-
-template <int TPR, int KMAX, bool PAD, bool FIX>
-__global__ __launch_bounds__(TPR ? TPR : 1024, (TPR == 0 && KMAX <= 4) ? 8 : 1) void rmsnorm_kernel(float *o, float *x, const float *weight, int dim, float eps) {
-  rms_row<TPR, KMAX, false, 0, PAD, FIX>(o, nullptr, nullptr, x, nullptr, weight, dim, eps);
-}
-
-template <int TPR, int KMAX, int QGS, bool PAD>
-__global__ __launch_bounds__(TPR) void rmsnorm_quantize_kernel(int8_t *q, float *q_s, float *x, const float *weight,
-                                                               int dim, float eps) {
-  rms_row<TPR, KMAX, false, QGS, PAD>(nullptr, q, q_s, x, nullptr, weight, dim, eps);
-}
-
-template <int TPR, int KMAX, int QGS, bool PAD>
-__global__ __launch_bounds__(TPR) void add_rmsnorm_quantize_kernel(int8_t *q, float *q_s, float *residual,
-                                                                   const float *add, const float *weight, int dim,
-                                                                   float eps) {
-  rms_row<TPR, KMAX, true, QGS, PAD>(nullptr, q, q_s, residual, add, weight, dim, eps);
-}
-
-// Chooses threads per row and float4 chunks per thread for dim <= 16384
-// (validated by the caller) and launches one workgroup per row.
-struct RowLaunch {
-  int rows, dim;
-  hipStream_t stream;
-  // the padded layout and DPP reduction: whole 32-float blocks, at most 64 KiB of LDS (5 bytes per element)
-  bool pad() const { return dim % 32 == 0 && dim <= 12288; }
-  // one float4 chunk per thread and k, all live: the fixed-length kernels
-  bool fits(int tpr, int kmax) const { return pad() && dim == 4 * tpr * kmax; }
-  size_t lds() const { return (size_t)(pad() ? dim + dim / 4 : dim) * sizeof(float); }
-};
-
-// Rows below 1024 floats take one wave each (up to 4 float4 chunks per lane)
-// when there are more than 2048 of them: 256-thread rows would then need more
-// than one round of the 8192 waves the GPU holds at once (256 CUs x 4 SIMDs x
-// 8), one-wave rows fit 8192 rows in one ([4096, 384]: 7.4 -> 5.8 us; [8192,
-// 896]: 21.9 -> 21.3 us).  Fewer rows keep the 256-thread row, whose loads
-// spread over four waves (up to 0.6 us faster from 64 to 2048 rows).
-template <template <int, int> class Op, typename... A>
-static void dispatch_rows(const RowLaunch &L, A... args) {
-  const bool wave_rows = L.rows > 2048;
-  if (L.dim <= 256)
-    Op<64, 1>::launch(L, args...);
-  else if (L.dim <= 512 && wave_rows)
-    Op<64, 2>::launch(L, args...);
-  else if (L.dim <= 768 && wave_rows)
-    Op<64, 3>::launch(L, args...);
-  else if (L.dim < 1024 && wave_rows)
-    Op<64, 4>::launch(L, args...);
-  else if (L.dim <= 1024)
-    Op<256, 1>::launch(L, args...);
-  else if (L.dim <= 2048)
-    Op<256, 2>::launch(L, args...);
-  else if (L.dim <= 4096)
-    Op<256, 4>::launch(L, args...);
-  else if (L.dim <= 8192)
-    Op<256, 8>::launch(L, args...);
-  else
-    Op<256, 16>::launch(L, args...);
-}
-
-template <int TPR, int KMAX>
-struct AddNormOp {
-  static void launch(const RowLaunch &L, float *o, float *residual, const float *add, const float *weight, float eps) {
-    auto go = [&](auto kernel) {
-      enqueue(kernel, dim3(L.rows), dim3(TPR), L.lds(), L.stream, o, residual, add, weight, L.dim, eps);
-    };
-    if (L.fits(TPR, KMAX))
-      go(fused_add_rmsnorm_kernel<TPR, KMAX, true, true>);
-    else if (L.pad())
-      go(fused_add_rmsnorm_kernel<TPR, KMAX, true, false>);
-    else
-      go(fused_add_rmsnorm_kernel<TPR, KMAX, false, false>);
+  constexpr int TPR = 256;
+  dim = 4 * TPR * KMAX;
+  extern __shared__ __attribute__((aligned(16))) float row[];
+  const int tid = threadIdx.x;
+  const size_t r = blockIdx.x;
+  float *xr = xin + r * (size_t)dim;
+  float4 x[KMAX], b[KMAX], w[KMAX];
+#pragma unroll
+  for (int k = 0; k < KMAX; ++k) {
+    const int i = 4 * (tid + k * TPR);
+    x[k] = ld_stream4(xr + i);
+    if constexpr (ADD) b[k] = ld_stream4(add + r * (size_t)dim + i);
   }
-};
-
-template <int TPR, int KMAX>
-struct NormOp {
-  static void launch(const RowLaunch &L, float *o, float *x, const float *weight, float eps) {
-    auto go = [&](auto kernel) { enqueue(kernel, dim3(L.rows), dim3(TPR), L.lds(), L.stream, o, x, weight, L.dim, eps); };
-    if (L.fits(TPR, KMAX))
-      go(rmsnorm_kernel<TPR, KMAX, true, true>);
-    else if (L.pad())
-      go(rmsnorm_kernel<TPR, KMAX, true, false>);
-    else
-      go(rmsnorm_kernel<TPR, KMAX, false, false>);
+  if constexpr (ADD) {
+#pragma unroll
+    for (int k = 0; k < KMAX; ++k) w[k] = *reinterpret_cast<const float4 *>(weight + 4 * (tid + k * TPR));
   }
-};
-
-template <int TPR, int KMAX>
-struct NormQ8Op {
-  static void launch(const RowLaunch &L, int8_t *q, float *q_s, float *x, const float *add, const float *weight,
-                     float eps, int gs) {
-    auto go_add = [&](auto kernel) {
-      enqueue(kernel, dim3(L.rows), dim3(TPR), L.lds(), L.stream, q, q_s, x, add, weight, L.dim, eps);
-    };
-    auto go = [&](auto kernel) {
-      enqueue(kernel, dim3(L.rows), dim3(TPR), L.lds(), L.stream, q, q_s, x, weight, L.dim, eps);
-    };
-    const bool pad = L.pad();
-    if (add) {
-      if (gs == 32)
-        pad ? go_add(add_rmsnorm_quantize_kernel<TPR, KMAX, 32, true>)
-            : go_add(add_rmsnorm_quantize_kernel<TPR, KMAX, 32, false>);
-      else
-        pad ? go_add(add_rmsnorm_quantize_kernel<TPR, KMAX, 64, true>)
-            : go_add(add_rmsnorm_quantize_kernel<TPR, KMAX, 64, false>);
-    } else {
-      if (gs == 32)
-        pad ? go(rmsnorm_quantize_kernel<TPR, KMAX, 32, true>) : go(rmsnorm_quantize_kernel<TPR, KMAX, 32, false>);
-      else
-        pad ? go(rmsnorm_quantize_kernel<TPR, KMAX, 64, true>) : go(rmsnorm_quantize_kernel<TPR, KMAX, 64, false>);
+#pragma unroll
+  for (int k = 0; k < KMAX; ++k) {
+    const int i = 4 * (tid + k * TPR);
+    if constexpr (ADD) {
+      x[k] = make_float4(x[k].x + b[k].x, x[k].y + b[k].y, x[k].z + b[k].z, x[k].w + b[k].w);
+      st_stream4(xr + i, x[k]);
     }
+    *reinterpret_cast<float4 *>(row + padded(tid + k * TPR)) = x[k];
   }
-};
-
-template <bool ADD, int TPR, int KMAX>
-static auto fixed_row_kernel() {
-  if constexpr (ADD)
-    return fused_add_rmsnorm_kernel<TPR, KMAX, true, true>;
-  else
-    return rmsnorm_kernel<TPR, KMAX, true, true>;
+  __syncthreads();
+  // floats 16..19 of the padded layout are padding: the scale goes there
+  if (tid < 64) {
+    const float s0 = rms_scale(padded_row_sumsq<8>(row, dim), (float)dim, eps);
+    if (tid == 0) row[16] = s0;
+  }
+  __syncthreads();
+  const float s = row[16];
+#pragma unroll
+  for (int k = 0; k < KMAX; ++k) {
+    const int i = 4 * (tid + k * TPR);
+    if constexpr (!ADD) w[k] = *reinterpret_cast<const float4 *>(weight + i);
+    st_stream4(o + r * (size_t)dim + i, make_float4((s * x[k].x) * w[k].x, (s * x[k].y) * w[k].y,
+                                                    (s * x[k].z) * w[k].z, (s * x[k].w) * w[k].w));
+  }
 }
 
-// The fixed-length row at the widths between and above the powers of two,
-// 1024 < dim <= 8192, dim % 256 == 0 (dim = 4 * threads * chunks): the shape
-// that measured fastest at [8192, dim] for the common model widths, compiled
-// in (2560, 3072, 3584, 3840, 5120, 8192: 1.5 to 2.5 points of the HBM peak
-// above the general kernel, 8192 even); a run-time thread count with 2
-// chunks per thread (1 where dim/4 is an odd multiple of 64) for the other
-// multiples of 256 up to 4096 and of 512 up to 8192 (whole waves, at most
-// 1024 threads).  2048 and 4096 keep the
-// dispatch_rows shapes, which measured best.  Returns false where none applies.
-template <bool ADD>
-static bool launch_fixed_row(const RowLaunch &L, float *o, float *x, const float *add, const float *weight,
-                             float eps) {
-  if (L.dim <= 1024 || L.dim > 8192 || L.dim % 256 || L.dim == 2048 || L.dim == 4096) return false;
-  auto go = [&](auto kernel, int tpr) {
-    if constexpr (ADD)
-      enqueue(kernel, dim3(L.rows), dim3(tpr), L.lds(), L.stream, o, x, add, weight, L.dim, eps);
-    else
-      enqueue(kernel, dim3(L.rows), dim3(tpr), L.lds(), L.stream, o, x, weight, L.dim, eps);
+// Calls go(tpr, kmax) with the shape as compile-time constants: kmax chunks per
+// thread, the fewest whole waves that hold dim floats.  False, and no call,
+// where that leaves more than the last chunk partly past the row's end
+// (rms_row tests only the last one) or no kernel of that size is built.
+template <int KMAX, int MIN_WAVES, int MAX_WAVES, typename Go>
+static bool with_threads(int dim, Go go) {
+  const int waves = (dim / 4 + 64 * KMAX - 1) / (64 * KMAX);
+  if (waves < MIN_WAVES || waves > MAX_WAVES || 64 * waves * (KMAX - 1) > dim / 4) return false;
+  using std::integral_constant;
+  constexpr integral_constant<int, KMAX> k{};
+  auto call = [&](auto tpr) {
+    constexpr int waves_c = decltype(tpr)::value / 64;
+    if constexpr (waves_c >= MIN_WAVES && waves_c <= MAX_WAVES) go(tpr, k);
   };
-  switch (L.dim) {
-    case 2560: go(fixed_row_kernel<ADD, 320, 2>(), 320); return true;
-    case 3072: go(fixed_row_kernel<ADD, 256, 3>(), 256); return true;
-    case 3584: go(fixed_row_kernel<ADD, 448, 2>(), 448); return true;
-    case 3840: go(fixed_row_kernel<ADD, 960, 1>(), 960); return true;
-    case 5120: go(fixed_row_kernel<ADD, 640, 2>(), 640); return true;
-    case 8192: go(fixed_row_kernel<ADD, 512, 4>(), 512); return true;
+  switch (waves) {
+    case 1: call(integral_constant<int, 64>{}); break;
+    case 2: call(integral_constant<int, 128>{}); break;
+    case 3: call(integral_constant<int, 192>{}); break;
+    case 4: call(integral_constant<int, 256>{}); break;
+    case 5: call(integral_constant<int, 320>{}); break;
+    case 6: call(integral_constant<int, 384>{}); break;
+    case 7: call(integral_constant<int, 448>{}); break;
+    case 8: call(integral_constant<int, 512>{}); break;
+    case 9: call(integral_constant<int, 576>{}); break;
+    case 10: call(integral_constant<int, 640>{}); break;
+    case 11: call(integral_constant<int, 704>{}); break;
+    case 12: call(integral_constant<int, 768>{}); break;
+    case 13: call(integral_constant<int, 832>{}); break;
+    case 14: call(integral_constant<int, 896>{}); break;
+    case 15: call(integral_constant<int, 960>{}); break;
+    default: call(integral_constant<int, 1024>{}); break;
   }
-  const int chunks = L.dim / 4;  // a multiple of 64: whole waves
-  if (chunks % 128 == 0 && chunks / 2 <= 1024)
-    go(fixed_row_kernel<ADD, 0, 2>(), chunks / 2);
-  else if (chunks <= 1024)
-    go(fixed_row_kernel<ADD, 0, 1>(), chunks);
-  else
-    return false;
   return true;
+}
+
+// At most one row per CU: what counts is a row's own latency.
+constexpr int kFewRows = 256;
+
+// The row's shape, each line from the times of [rows, dim] on one MI355X:
+//  - at most 256 rows: one chunk per thread up to 1024 floats, two up to 8192,
+//    four beyond and at 4096 and 8192 (fewer waves to gather at the barriers:
+//    [8, 4096] 3.03 us against 3.22 with two);
+//  - 1024, 2048, 3072, 4096: rmsnorm_fixed_row_kernel;
+//  - above 2048 rows, below 1024 floats: a wave per row, so that more rows are
+//    resident ([3500, 896] RMSNorm 5.2 us against 6.8 with four waves; with
+//    the add the wave's registers hold only up to 768);
+//  - one chunk per thread up to 1024 floats (2048 with the add, or up to four
+//    rows per CU: [1000, 1984] RMSNorm 4.0 us against 4.3);
+//  - two chunks up to 8192, four beyond (two rows of 1024 threads per CU);
+//  - eight chunks where fewer threads per row measured faster: with the add at
+//    up to two rows per CU ([500, 5376] 8.9 us against 9.8 with two chunks),
+//    without it at two to four ([1000, 5376] 7.7 against 10.6).
+template <bool ADD>
+static void launch_row(float *o, float *x, const float *add, const float *weight, int rows, int dim, float eps,
+                       hipStream_t stream) {
+  using std::integral_constant;
+  auto go = [&](auto tpr, auto kmax, auto leftover, auto few) {
+    constexpr int TPR = decltype(tpr)::value, K = decltype(kmax)::value;
+    constexpr bool LEFT = decltype(leftover)::value, FEW = decltype(few)::value;
+    enqueue(rmsnorm_row_kernel<TPR, K, ADD, LEFT, FEW>, dim3(rows), dim3(TPR),
+            ChainLayout<TPR, K, LEFT, row_chain_u(K, FEW)>::kBytes, stream, o, x, add, weight, dim, eps);
+  };
+  if (dim % 32) {
+    auto left = [&](auto tpr, auto kmax) { go(tpr, kmax, std::true_type{}, std::false_type{}); };
+    if (dim <= 256)
+      left(integral_constant<int, 64>{}, integral_constant<int, 1>{});
+    else if (dim <= 1024)
+      left(integral_constant<int, 256>{}, integral_constant<int, 1>{});
+    else if (dim <= 4096)
+      left(integral_constant<int, 512>{}, integral_constant<int, 2>{});
+    else if (dim <= 8192)
+      left(integral_constant<int, 1024>{}, integral_constant<int, 2>{});
+    else
+      left(integral_constant<int, 1024>{}, integral_constant<int, 4>{});
+    return;
+  }
+  auto few = [&](auto tpr, auto kmax) { go(tpr, kmax, std::false_type{}, std::true_type{}); };
+  auto many = [&](auto tpr, auto kmax) { go(tpr, kmax, std::false_type{}, std::false_type{}); };
+  if (rows <= kFewRows) {
+    if (dim <= 1024)
+      with_threads<1, 1, 4>(dim, few);
+    else if (dim % 4096 && dim <= 8192)
+      with_threads<2, 3, 16>(dim, few);
+    else
+      with_threads<4, 4, 16>(dim, few);
+    return;
+  }
+  auto fixed = [&](auto kmax) {
+    enqueue(rmsnorm_fixed_row_kernel<decltype(kmax)::value, ADD>, dim3(rows), dim3(256),
+            (unsigned)(dim + dim / 4) * 4u, stream, o, x, add, weight, dim, eps);
+  };
+  switch (dim) {
+    case 1024: return fixed(integral_constant<int, 1>{});
+    case 2048: return fixed(integral_constant<int, 2>{});
+    case 3072: return fixed(integral_constant<int, 3>{});
+    case 4096: return fixed(integral_constant<int, 4>{});
+  }
+  const bool two_per_cu = rows <= 2 * kFewRows, four_per_cu = rows <= 4 * kFewRows;
+  if (rows > 2048 && dim > 256 && dim <= (ADD ? 768 : 1024)) {
+    if (dim <= 512)
+      many(integral_constant<int, 64>{}, integral_constant<int, 2>{});
+    else if (dim <= 768)
+      many(integral_constant<int, 64>{}, integral_constant<int, 3>{});
+    else
+      many(integral_constant<int, 64>{}, integral_constant<int, 4>{});
+    return;
+  }
+  if (dim <= 1024 || (dim <= 2048 && (ADD || four_per_cu)))
+    with_threads<1, 1, 8>(dim, many);
+  else if (dim <= 4096)
+    with_threads<2, 3, 8>(dim, many);
+  else if ((ADD ? two_per_cu : four_per_cu && !two_per_cu && dim < 8192) && with_threads<8, 3, 8>(dim, many))
+    return;
+  else if (dim < 8192)
+    with_threads<2, 9, 16>(dim, many);
+  else
+    with_threads<4, 8, 16>(dim, many);
 }
 
 void launch_fused_add_rmsnorm(float *o, float *residual, const float *add, const float *weight, int rows, int dim,
                               float eps, hipStream_t stream) {
-  const RowLaunch L{rows, dim, stream};
-  if (!launch_fixed_row<true>(L, o, residual, add, weight, eps))
-    dispatch_rows<AddNormOp>(L, o, residual, add, weight, eps);
+  launch_row<true>(o, residual, add, weight, rows, dim, eps, stream);
 }
 
 void launch_rmsnorm(float *o, const float *x, const float *weight, int rows, int dim, float eps, hipStream_t stream) {
-  const RowLaunch L{rows, dim, stream};
-  if (!launch_fixed_row<false>(L, o, const_cast<float *>(x), nullptr, weight, eps))
-    dispatch_rows<NormOp>(L, o, const_cast<float *>(x), weight, eps);
+  launch_row<false>(o, const_cast<float *>(x), nullptr, weight, rows, dim, eps, stream);
+}
+
+template <int QGS, bool ADD>
+static void launch_q8_row(int8_t *q, float *q_s, float *x, const float *add, const float *weight, int rows, int dim,
+                          float eps, hipStream_t stream) {
+  auto go = [&](auto tpr, auto kmax, auto few) {
+    constexpr int TPR = decltype(tpr)::value, K = decltype(kmax)::value;
+    constexpr bool FEW = decltype(few)::value;
+    enqueue(rmsnorm_q8_row_kernel<TPR, K, QGS, ADD, FEW>, dim3(rows), dim3(TPR),
+            ChainLayout<TPR, K, false, row_chain_u(K, FEW)>::kBytes, stream, q, q_s, x, add, weight, dim, eps);
+  };
+  auto few = [&](auto tpr, auto kmax) { go(tpr, kmax, std::true_type{}); };
+  auto many = [&](auto tpr, auto kmax) { go(tpr, kmax, std::false_type{}); };
+  if (rows > 2048 && dim > 256 && dim <= 512)
+    many(std::integral_constant<int, 64>{}, std::integral_constant<int, 2>{});
+  else if (dim <= 4096)
+    with_threads<1, 1, 16>(dim, few);
+  else if (dim <= 8192)
+    with_threads<2, 9, 16>(dim, few);
+  else if (rows <= kFewRows)
+    with_threads<4, 9, 16>(dim, few);
+  else
+    with_threads<4, 9, 16>(dim, many);
 }
 
 void launch_rmsnorm_quantize(int8_t *q, float *q_s, float *x, const float *add, const float *weight, int rows,
                              int dim, int gs, float eps, hipStream_t stream) {
+  // At most one row per CU takes the row kernel, whose chain is shorter and whose
+  // results need no second pass through LDS ([1, 2304] 2.84 -> 2.21 us with the
+  // add, [8, 4096] 3.49 -> 3.36); beyond that norm_q8_row16_kernel's quantizer,
+  // with a quarter of the instructions, wins ([512, 2560] 5.31 us against 5.59).
   // The 16-elements-per-thread kernel needs the 32 chain lanes (dim >= 512), whole
   // 32-element blocks, 16-byte aligned codes and at most 64 KiB of LDS (5 bytes per element).
-  if (dim % 32 == 0 && dim >= 512 && dim <= 12288 && ((uintptr_t)q & 15u) == 0) {
+    if (rows > kFewRows && dim % 32 == 0 && dim >= 512 && dim <= 12288 && ((uintptr_t)q & 15u) == 0) {
     const dim3 grid(rows), block(dim / 16);
     const unsigned lds = (unsigned)(dim + dim / 4) * sizeof(float);
     auto go = [&](auto kernel) { enqueue(kernel, grid, block, lds, stream, q, q_s, x, add, weight, dim, eps); };
@@ -563,7 +698,12 @@ void launch_rmsnorm_quantize(int8_t *q, float *q_s, float *x, const float *add, 
     }
     return;
   }
-  dispatch_rows<NormQ8Op>(RowLaunch{rows, dim, stream}, q, q_s, x, add, weight, eps, gs);
+  if (add)
+    gs == 32 ? launch_q8_row<32, true>(q, q_s, x, add, weight, rows, dim, eps, stream)
+             : launch_q8_row<64, true>(q, q_s, x, add, weight, rows, dim, eps, stream);
+  else
+    gs == 32 ? launch_q8_row<32, false>(q, q_s, x, add, weight, rows, dim, eps, stream)
+             : launch_q8_row<64, false>(q, q_s, x, add, weight, rows, dim, eps, stream);
 }
 
 }  // namespace v7g

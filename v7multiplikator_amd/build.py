@@ -88,6 +88,31 @@ def build_library(verbose: bool = False) -> str:
     return LIB
 
 
+def build_native(verbose: bool = False) -> str:
+    """Builds native/ops_native.cpp, the CPython module _ops_native that checks and launches the accepted calls of
+    ops, against the installed torch (host only, g++); returns its path."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    src = os.path.join(PKG, "native", "ops_native.cpp")
+    out = os.path.join(PKG, "_ops_native.so")
+    lib_dirs = [os.path.join(os.path.dirname(torch.__file__), "lib")]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[a for p in cpp_extension.include_paths() for a in ("-isystem", p)],
+           "-isystem", sysconfig.get_paths()["include"], "-o", out + ".tmp", src,
+           *[f"-L{d}" for d in lib_dirs], "-lc10", "-ltorch_cpu", "-ltorch_python"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed ({res.returncode}):\n{res.stdout}{res.stderr}")
+    os.replace(out + ".tmp", out)
+    return out
+
+
 def build_loadtest(verbose: bool = False) -> str:
     """Builds the C++ harness csrc/v7g_loadtest.cpp (host only, dlopens libv7g.so)."""
     src = os.path.join(CSRC, "v7g_loadtest.cpp")
@@ -134,6 +159,7 @@ def build_test_shim(verbose: bool = False) -> str:
 
 if __name__ == "__main__":
     print(build_library(verbose=True))
+    print(build_native(verbose=True))
     if os.path.exists(os.path.join(CSRC, "v7g_loadtest.cpp")):
         print(build_loadtest(verbose=True))
     sys.exit(0)

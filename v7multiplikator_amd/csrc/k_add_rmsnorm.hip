@@ -585,6 +585,19 @@ static bool with_threads(int dim, Go go) {
   return true;
 }
 
+// Calls launch(first row, rows) over all rows, one workgroup of tpr threads per
+// row.  HIP refuses a grid dimension of 2^32 threads or more, so more rows than
+// that go in several launches.
+template <typename Launch>
+static void by_rows(int rows, int tpr, Launch launch) {
+  const int most = (int)(0xFFFFFFFFu / (unsigned)tpr);
+  for (int first = 0; first < rows;) {
+    const int n = rows - first < most ? rows - first : most;
+    launch(first, n);
+    first += n;
+  }
+}
+
 // At most one row per CU: what counts is a row's own latency.
 constexpr int kFewRows = 256;
 
@@ -603,43 +616,42 @@ constexpr int kFewRows = 256;
 //    up to two rows per CU ([500, 5376] 8.9 us against 9.8 with two chunks),
 //    without it at two to four ([1000, 5376] 7.7 against 10.6).
 template <bool ADD>
-static void launch_row(float *o, float *x, const float *add, const float *weight, int rows, int dim, float eps,
+static bool launch_row(float *o, float *x, const float *add, const float *weight, int rows, int dim, float eps,
                        hipStream_t stream) {
   using std::integral_constant;
   auto go = [&](auto tpr, auto kmax, auto leftover, auto few) {
     constexpr int TPR = decltype(tpr)::value, K = decltype(kmax)::value;
     constexpr bool LEFT = decltype(leftover)::value, FEW = decltype(few)::value;
-    enqueue(rmsnorm_row_kernel<TPR, K, ADD, LEFT, FEW>, dim3(rows), dim3(TPR),
-            ChainLayout<TPR, K, LEFT, row_chain_u(K, FEW)>::kBytes, stream, o, x, add, weight, dim, eps);
+    by_rows(rows, TPR, [&](int first, int n) {
+      const size_t at = (size_t)first * (size_t)dim;
+      enqueue(rmsnorm_row_kernel<TPR, K, ADD, LEFT, FEW>, dim3(n), dim3(TPR),
+              ChainLayout<TPR, K, LEFT, row_chain_u(K, FEW)>::kBytes, stream, o + at, x + at, ADD ? add + at : add,
+              weight, dim, eps);
+    });
+    return true;
   };
   if (dim % 32) {
-    auto left = [&](auto tpr, auto kmax) { go(tpr, kmax, std::true_type{}, std::false_type{}); };
-    if (dim <= 256)
-      left(integral_constant<int, 64>{}, integral_constant<int, 1>{});
-    else if (dim <= 1024)
-      left(integral_constant<int, 256>{}, integral_constant<int, 1>{});
-    else if (dim <= 4096)
-      left(integral_constant<int, 512>{}, integral_constant<int, 2>{});
-    else if (dim <= 8192)
-      left(integral_constant<int, 1024>{}, integral_constant<int, 2>{});
-    else
-      left(integral_constant<int, 1024>{}, integral_constant<int, 4>{});
-    return;
+    auto left = [&](auto tpr, auto kmax) { return go(tpr, kmax, std::true_type{}, std::false_type{}); };
+    if (dim <= 256) return left(integral_constant<int, 64>{}, integral_constant<int, 1>{});
+    if (dim <= 1024) return left(integral_constant<int, 256>{}, integral_constant<int, 1>{});
+    if (dim <= 4096) return left(integral_constant<int, 512>{}, integral_constant<int, 2>{});
+    if (dim <= 8192) return left(integral_constant<int, 1024>{}, integral_constant<int, 2>{});
+    return left(integral_constant<int, 1024>{}, integral_constant<int, 4>{});
   }
-  auto few = [&](auto tpr, auto kmax) { go(tpr, kmax, std::false_type{}, std::true_type{}); };
-  auto many = [&](auto tpr, auto kmax) { go(tpr, kmax, std::false_type{}, std::false_type{}); };
+  auto few = [&](auto tpr, auto kmax) { return go(tpr, kmax, std::false_type{}, std::true_type{}); };
+  auto many = [&](auto tpr, auto kmax) { return go(tpr, kmax, std::false_type{}, std::false_type{}); };
   if (rows <= kFewRows) {
-    if (dim <= 1024)
-      with_threads<1, 1, 4>(dim, few);
-    else if (dim % 4096 && dim <= 8192)
-      with_threads<2, 3, 16>(dim, few);
-    else
-      with_threads<4, 4, 16>(dim, few);
-    return;
+    if (dim <= 1024) return with_threads<1, 1, 4>(dim, few);
+    if (dim % 4096 && dim <= 8192) return with_threads<2, 3, 16>(dim, few);
+    return with_threads<4, 4, 16>(dim, few);
   }
   auto fixed = [&](auto kmax) {
-    enqueue(rmsnorm_fixed_row_kernel<decltype(kmax)::value, ADD>, dim3(rows), dim3(256),
-            (unsigned)(dim + dim / 4) * 4u, stream, o, x, add, weight, dim, eps);
+    by_rows(rows, 256, [&](int first, int n) {
+      const size_t at = (size_t)first * (size_t)dim;
+      enqueue(rmsnorm_fixed_row_kernel<decltype(kmax)::value, ADD>, dim3(n), dim3(256),
+              (unsigned)(dim + dim / 4) * 4u, stream, o + at, x + at, ADD ? add + at : add, weight, dim, eps);
+    });
+    return true;
   };
   switch (dim) {
     case 1024: return fixed(integral_constant<int, 1>{});
@@ -649,59 +661,49 @@ static void launch_row(float *o, float *x, const float *add, const float *weight
   }
   const bool two_per_cu = rows <= 2 * kFewRows, four_per_cu = rows <= 4 * kFewRows;
   if (rows > 2048 && dim > 256 && dim <= (ADD ? 768 : 1024)) {
-    if (dim <= 512)
-      many(integral_constant<int, 64>{}, integral_constant<int, 2>{});
-    else if (dim <= 768)
-      many(integral_constant<int, 64>{}, integral_constant<int, 3>{});
-    else
-      many(integral_constant<int, 64>{}, integral_constant<int, 4>{});
-    return;
+    if (dim <= 512) return many(integral_constant<int, 64>{}, integral_constant<int, 2>{});
+    if (dim <= 768) return many(integral_constant<int, 64>{}, integral_constant<int, 3>{});
+    return many(integral_constant<int, 64>{}, integral_constant<int, 4>{});
   }
-  if (dim <= 1024 || (dim <= 2048 && (ADD || four_per_cu)))
-    with_threads<1, 1, 8>(dim, many);
-  else if (dim <= 4096)
-    with_threads<2, 3, 8>(dim, many);
-  else if ((ADD ? two_per_cu : four_per_cu && !two_per_cu && dim < 8192) && with_threads<8, 3, 8>(dim, many))
-    return;
-  else if (dim < 8192)
-    with_threads<2, 9, 16>(dim, many);
-  else
-    with_threads<4, 8, 16>(dim, many);
+  if (dim <= 1024 || (dim <= 2048 && (ADD || four_per_cu))) return with_threads<1, 1, 8>(dim, many);
+  if (dim <= 4096) return with_threads<2, 3, 8>(dim, many);
+  if ((ADD ? two_per_cu : four_per_cu && !two_per_cu && dim < 8192) && with_threads<8, 3, 8>(dim, many)) return true;
+  return dim < 8192 ? with_threads<2, 9, 16>(dim, many) : with_threads<4, 8, 16>(dim, many);
 }
 
-void launch_fused_add_rmsnorm(float *o, float *residual, const float *add, const float *weight, int rows, int dim,
+bool launch_fused_add_rmsnorm(float *o, float *residual, const float *add, const float *weight, int rows, int dim,
                               float eps, hipStream_t stream) {
-  launch_row<true>(o, residual, add, weight, rows, dim, eps, stream);
+  return launch_row<true>(o, residual, add, weight, rows, dim, eps, stream);
 }
 
-void launch_rmsnorm(float *o, const float *x, const float *weight, int rows, int dim, float eps, hipStream_t stream) {
-  launch_row<false>(o, const_cast<float *>(x), nullptr, weight, rows, dim, eps, stream);
+bool launch_rmsnorm(float *o, const float *x, const float *weight, int rows, int dim, float eps, hipStream_t stream) {
+  return launch_row<false>(o, const_cast<float *>(x), nullptr, weight, rows, dim, eps, stream);
 }
 
 template <int QGS, bool ADD>
-static void launch_q8_row(int8_t *q, float *q_s, float *x, const float *add, const float *weight, int rows, int dim,
+static bool launch_q8_row(int8_t *q, float *q_s, float *x, const float *add, const float *weight, int rows, int dim,
                           float eps, hipStream_t stream) {
   auto go = [&](auto tpr, auto kmax, auto few) {
     constexpr int TPR = decltype(tpr)::value, K = decltype(kmax)::value;
     constexpr bool FEW = decltype(few)::value;
-    enqueue(rmsnorm_q8_row_kernel<TPR, K, QGS, ADD, FEW>, dim3(rows), dim3(TPR),
-            ChainLayout<TPR, K, false, row_chain_u(K, FEW)>::kBytes, stream, q, q_s, x, add, weight, dim, eps);
+    by_rows(rows, TPR, [&](int first, int n) {
+      const size_t at = (size_t)first * (size_t)dim;
+      enqueue(rmsnorm_q8_row_kernel<TPR, K, QGS, ADD, FEW>, dim3(n), dim3(TPR),
+              ChainLayout<TPR, K, false, row_chain_u(K, FEW)>::kBytes, stream, q + at, q_s + at / QGS, x + at,
+              ADD ? add + at : add, weight, dim, eps);
+    });
+    return true;
   };
-  auto few = [&](auto tpr, auto kmax) { go(tpr, kmax, std::true_type{}); };
-  auto many = [&](auto tpr, auto kmax) { go(tpr, kmax, std::false_type{}); };
+  auto few = [&](auto tpr, auto kmax) { return go(tpr, kmax, std::true_type{}); };
+  auto many = [&](auto tpr, auto kmax) { return go(tpr, kmax, std::false_type{}); };
   if (rows > 2048 && dim > 256 && dim <= 512)
-    many(std::integral_constant<int, 64>{}, std::integral_constant<int, 2>{});
-  else if (dim <= 4096)
-    with_threads<1, 1, 16>(dim, few);
-  else if (dim <= 8192)
-    with_threads<2, 9, 16>(dim, few);
-  else if (rows <= kFewRows)
-    with_threads<4, 9, 16>(dim, few);
-  else
-    with_threads<4, 9, 16>(dim, many);
+    return many(std::integral_constant<int, 64>{}, std::integral_constant<int, 2>{});
+  if (dim <= 4096) return with_threads<1, 1, 16>(dim, few);
+  if (dim <= 8192) return with_threads<2, 9, 16>(dim, few);
+  return rows <= kFewRows ? with_threads<4, 9, 16>(dim, few) : with_threads<4, 9, 16>(dim, many);
 }
 
-void launch_rmsnorm_quantize(int8_t *q, float *q_s, float *x, const float *add, const float *weight, int rows,
+bool launch_rmsnorm_quantize(int8_t *q, float *q_s, float *x, const float *add, const float *weight, int rows,
                              int dim, int gs, float eps, hipStream_t stream) {
   // At most one row per CU takes the row kernel, whose chain is shorter and whose
   // results need no second pass through LDS ([1, 2304] 2.84 -> 2.21 us with the
@@ -709,7 +711,7 @@ void launch_rmsnorm_quantize(int8_t *q, float *q_s, float *x, const float *add, 
   // with a quarter of the instructions, wins ([512, 2560] 5.31 us against 5.59).
   // The 16-elements-per-thread kernel needs the 32 chain lanes (dim >= 512), whole
   // 32-element blocks, 16-byte aligned codes and at most 64 KiB of LDS (5 bytes per element).
-    if (rows > kFewRows && dim % 32 == 0 && dim >= 512 && dim <= 12288 && ((uintptr_t)q & 15u) == 0) {
+  if (rows > kFewRows && dim % 32 == 0 && dim >= 512 && dim <= 12288 && ((uintptr_t)q & 15u) == 0) {
     const dim3 grid(rows), block(dim / 16);
     const unsigned lds = (unsigned)(dim + dim / 4) * sizeof(float);
     auto go = [&](auto kernel) { enqueue(kernel, grid, block, lds, stream, q, q_s, x, add, weight, dim, eps); };
@@ -735,14 +737,13 @@ void launch_rmsnorm_quantize(int8_t *q, float *q_s, float *x, const float *add, 
       case 8192: go_tpb(std::integral_constant<int, 512>{}); break;
       default: go_tpb(std::integral_constant<int, 0>{}); break;
     }
-    return;
+    return true;
   }
   if (add)
-    gs == 32 ? launch_q8_row<32, true>(q, q_s, x, add, weight, rows, dim, eps, stream)
-             : launch_q8_row<64, true>(q, q_s, x, add, weight, rows, dim, eps, stream);
-  else
-    gs == 32 ? launch_q8_row<32, false>(q, q_s, x, add, weight, rows, dim, eps, stream)
-             : launch_q8_row<64, false>(q, q_s, x, add, weight, rows, dim, eps, stream);
+    return gs == 32 ? launch_q8_row<32, true>(q, q_s, x, add, weight, rows, dim, eps, stream)
+                    : launch_q8_row<64, true>(q, q_s, x, add, weight, rows, dim, eps, stream);
+  return gs == 32 ? launch_q8_row<32, false>(q, q_s, x, add, weight, rows, dim, eps, stream)
+                  : launch_q8_row<64, false>(q, q_s, x, add, weight, rows, dim, eps, stream);
 }
 
 }  // namespace v7g

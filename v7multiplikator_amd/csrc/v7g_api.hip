@@ -62,9 +62,10 @@ int fail(int code) {
 
 // Called after the launches of every launching entry: also disarms the timing
 // events, which cover that one call.
-int check_launch() {
+int check_launch(bool launched = true) {
   v7g::launch_events() = v7g::LaunchEvents{};
   hipError_t e = hipGetLastError();
+  if (!launched) return fail(V7G_ERR_SHAPE);  // no kernel is built for an accepted shape
   return e == hipSuccess ? V7G_OK : fail(V7G_ERR_HIP);
 }
 
@@ -448,8 +449,7 @@ int v7g_fused_add_rmsnorm(float *o, float *residual, const float *add, const flo
   if (rc) return fail(rc);
   if (rows == 0) return V7G_OK;
   if (int pc = check_ptrs({o, residual, add, weight})) return fail(pc);
-  v7g::launch_fused_add_rmsnorm(o, residual, add, weight, rows, dim, eps, stream());
-  return check_launch();
+  return check_launch(v7g::launch_fused_add_rmsnorm(o, residual, add, weight, rows, dim, eps, stream()));
 }
 
 int v7g_rmsnorm(float *o, const float *x, const float *weight, int rows, int dim, float eps) {
@@ -464,8 +464,7 @@ int v7g_rmsnorm(float *o, const float *x, const float *weight, int rows, int dim
     if ((o != x && overlap(O, X)) || overlap(O, W)) return fail(V7G_ERR_ALIAS);  // o == x: in place
   }
   if (int pc = check_ptrs({o, x, weight})) return fail(pc);
-  v7g::launch_rmsnorm(o, x, weight, rows, dim, eps, stream());
-  return check_launch();
+  return check_launch(v7g::launch_rmsnorm(o, x, weight, rows, dim, eps, stream()));
 }
 
 static int check_norm_q8(const int8_t *out_q, const float *out_s, const float *x, const float *weight, int rows,
@@ -494,8 +493,8 @@ int v7g_rmsnorm_quantize(int8_t *out_q, float *out_s, const float *x, const floa
   if (rc) return fail(rc);
   if (rows == 0) return V7G_OK;
   if (int pc = check_ptrs({out_q, out_s, x, weight})) return fail(pc);
-  v7g::launch_rmsnorm_quantize(out_q, out_s, const_cast<float *>(x), nullptr, weight, rows, dim, gs, eps, stream());
-  return check_launch();
+  return check_launch(v7g::launch_rmsnorm_quantize(out_q, out_s, const_cast<float *>(x), nullptr, weight, rows, dim, gs,
+                                                   eps, stream()));
 }
 
 int v7g_add_rmsnorm_quantize(int8_t *out_q, float *out_s, float *residual, const float *add, const float *weight,
@@ -507,8 +506,8 @@ int v7g_add_rmsnorm_quantize(int8_t *out_q, float *out_s, float *residual, const
   if (rc) return fail(rc);
   if (rows == 0) return V7G_OK;
   if (int pc = check_ptrs({out_q, out_s, residual, add, weight})) return fail(pc);
-  v7g::launch_rmsnorm_quantize(out_q, out_s, residual, add, weight, rows, dim, gs, eps, stream());
-  return check_launch();
+  return check_launch(
+      v7g::launch_rmsnorm_quantize(out_q, out_s, residual, add, weight, rows, dim, gs, eps, stream()));
 }
 
 int v7g_add_inplace(float *x, const float *y, long long n) {

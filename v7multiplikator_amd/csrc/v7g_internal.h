@@ -30,15 +30,16 @@ inline void enqueue(void (*kernel)(KArgs...), dim3 grid, dim3 block, unsigned ld
 void launch_embedding_gather(float *out, const int32_t *ids, int n_tokens, const int8_t *table_q,
                              const float *table_s, int dim, int vocab, hipStream_t stream);
 
-void launch_fused_add_rmsnorm(float *o, float *residual, const float *add, const float *weight, int rows, int dim,
+// The three row launchers answer false, having launched nothing, for a shape no kernel is built for.
+bool launch_fused_add_rmsnorm(float *o, float *residual, const float *add, const float *weight, int rows, int dim,
                               float eps, hipStream_t stream);
 
 // v7s_rmsnorm over rows x dim (dim % 32 == 0, <= 16384); o may alias x.
-void launch_rmsnorm(float *o, const float *x, const float *weight, int rows, int dim, float eps, hipStream_t stream);
+bool launch_rmsnorm(float *o, const float *x, const float *weight, int rows, int dim, float eps, hipStream_t stream);
 
 // RMSNorm -> Q8 over rows x dim (dim % gs == 0, gs 32 or 64); with add, x is a
 // residual updated in place as x + add first (add_inplace fused in front).
-void launch_rmsnorm_quantize(int8_t *q, float *q_s, float *x, const float *add, const float *weight, int rows,
+bool launch_rmsnorm_quantize(int8_t *q, float *q_s, float *x, const float *add, const float *weight, int rows,
                              int dim, int gs, float eps, hipStream_t stream);
 
 // x += y over n floats (n % 4 == 0 on the vector path; any n).

@@ -81,27 +81,31 @@ static void check(const char *op, int rows, int dim, int gs, unsigned elem, Call
     if (l.out != kBase + (unsigned long long)done * dim * elem) fault("rows out of order", op, rows, dim, gs, n.c_str());
     done += l.grid.x;
     const size_t chain = n.find("rmsnorm_row_kernelI"), q8 = n.find("rmsnorm_q8_row_kernelI"),
-                 fixed = n.find("rmsnorm_fixed_row_kernelI"), row16 = n.find("norm_q8_row16_kernelI");
+                 pad = n.find("padded_row_kernelI"), row16 = n.find("norm_q8_row16_kernelI");
     if (row16 != std::string::npos) {
       if (l.block.x * 16 != (unsigned)dim || l.lds < 5u * dim) fault("row16 shape", op, rows, dim, gs, n.c_str());
       continue;
     }
-    if (fixed != std::string::npos) {
-      const long kmax = ints_of(n, fixed)[0];
-      if (l.block.x != 256 || dim != 1024 * kmax || l.lds < 5u * dim) fault("fixed shape", op, rows, dim, gs, n.c_str());
-      continue;
-    }
-    const size_t at = q8 != std::string::npos ? q8 : chain;
+    const bool padded = pad != std::string::npos;
+    const size_t at = padded ? pad : q8 != std::string::npos ? q8 : chain;
     if (at == std::string::npos) {
       fault("unknown kernel", op, rows, dim, gs, n.c_str());
       continue;
     }
     const std::vector<long> t = ints_of(n, at);  // TPR, KMAX, ...
     const long tpr = t[0], kmax = t[1];
-    const bool left = q8 == std::string::npos && t[3];
     if (l.block.x != (unsigned)tpr || 4 * tpr * kmax < dim) fault("row does not fit", op, rows, dim, gs, n.c_str());
-    if (left != (dim % 32 != 0)) fault("leftover blocks", op, rows, dim, gs, n.c_str());
-    if (!left && 4 * tpr * (kmax - 1) > dim) fault("more than the last chunk past the row", op, rows, dim, gs, n.c_str());
+    if (padded) {
+      const bool fix = t[3], left = t[4];
+      const int m = dim / 4 - 1;
+      if ((fix && dim != 4 * tpr * kmax) || left != (dim % 32 != 0) || l.lds < 4u * (4 * (m + (m >> 2)) + 4) ||
+          l.lds < 80)
+        fault("padded shape", op, rows, dim, gs, n.c_str());
+    } else {
+      const bool left = q8 == std::string::npos && t[3];
+      if (left != (dim % 32 != 0)) fault("leftover blocks", op, rows, dim, gs, n.c_str());
+      if (!left && 4 * tpr * (kmax - 1) > dim) fault("more than the last chunk past the row", op, rows, dim, gs, n.c_str());
+    }
   }
   if (done != rows) fault("rows missing or twice", op, rows, dim, gs, "");
 }

@@ -18,7 +18,7 @@
 // FMA chains, chain by chain (ChainLayout), and reduce them with DPP row
 // shifts in the (A+B)+(C+D) + HADD_YMM pairing.
 // Bound: many rows by HBM ([8192, 4096] add+RMSNorm 85-86 us, 79% of the peak;
-// [1000, 16384] 53.2 -> 46.2 us with 1024 threads per row in place of 256); few
+// [1000, 16384] 50.5 -> 46.5 us with 1024 threads per row in place of 256); few
 // rows by latency: the loads, the chain (128 dependent FMAs at 4096 floats),
 // the scale's divisions and square root, the stores ([8, 4096] RMSNorm 3.29 ->
 // 2.67 us, add+RMSNorm -> Q8 3.49 -> 3.36, [8, 5376] add+RMSNorm 5.4 -> 3.4).
@@ -72,7 +72,7 @@ __device__ __forceinline__ float chain_reduce(float acc) {
 // [2000, 3840] 10.9 -> 10.3, [300, 2560] 3.88 -> 3.66), else the plain loop, which
 // the compiler batches by 16 (the three-set form with run-time bounds: 2-3%
 // slower at 576, 1088, 1536 and 7808, 1-2% faster at 832 and 2304).
-template <int U, bool RING>
+template <int U, bool RING, bool LEFT = false>
 __device__ __forceinline__ float padded_row_sumsq(const float *row, int dim) {
   const int lane = __lane_id();
   float acc = 0.0f;
@@ -81,7 +81,18 @@ __device__ __forceinline__ float padded_row_sumsq(const float *row, int dim) {
     // element 32g + v sits at float 40g + v + 4*(v >> 4)
     const float *p = row + v + 4 * (v >> 4);
     const int steps = dim >> 5;
-    if (steps % (2 * U) == 0) {
+    if constexpr (LEFT) {
+      // the (dim/8) % 4 leftover blocks, all into A; element 8*left + 32g + v is then at
+      // float 40g + 8*left + v + 4*((2*left + (v >> 2)) >> 2)
+      const int left = (dim >> 3) & 3;
+      if (v < 8)
+        for (int b = 0; b < left; ++b) {
+          const float e = row[8 * b + v + 4 * ((2 * b + (v >> 2)) >> 2)];
+          acc = __builtin_fmaf(e, e, acc);
+        }
+      p = row + 8 * left + v + 4 * ((2 * left + (v >> 2)) >> 2);
+    }
+    if (steps % (2 * U) == 0 && (!LEFT || steps > 0)) {
       // Two register sets of U chain elements: the LDS reads of one set are
       // in flight while the FMAs consume the other, so the chain waits on
       // LDS once instead of once per U steps.  Same FMAs, same order.  The
@@ -242,10 +253,10 @@ __device__ __forceinline__ float chain_sumsq(const float *row) {
 // stores predicated (a branch around a load would put a wait at its merge).
 // When the weights are requested (vector memory operations retire in issue
 // order, so a weight load behind the residual's stores waits for them):
-//  - FEW, at most one row per CU: once the row is staged, ahead of the
-//    residual's stores, so that they travel during the chain and delay neither
-//    the row nor the result ([1, 8192] add+RMSNorm 4.85 -> 4.02 us, with the
-//    chain's new layout);
+//  - FEW, at most one row per CU and the shapes of more rows that launch_row and
+//    launch_q8_row name: once the row is staged, ahead of the residual's stores, so
+//    that they travel during the chain and delay neither the row nor the result
+//    ([1, 8192] add+RMSNorm 4.85 -> 4.02 us, with the chain's new layout);
 //  - many rows, ADD: right behind the row's loads;
 //  - many rows without ADD: after the chain, so that the other rows on the CU
 //    get their loads first ([1024, 4096] 6.9 -> 6.2 us); with four and more
@@ -392,9 +403,10 @@ __device__ __forceinline__ void rms_row(float *o, int8_t *q, float *q_s, float *
 // the scale and reciprocal are computed once per 16 elements, and the 16
 // codes leave as one 16-byte store.  The fused-add form writes the updated
 // residual back with the loads' layout.  Same operations and order as
-// rms_row, so the same bits; about 10% less time at [8192, 4096] than
-// rms_row, whose 4-element-per-lane quantizer and lane-exchange reduction
-// made the kernel issue-bound.  The LDS array is declared 16-byte aligned:
+// rms_row, so the same bits; with many rows less time than rms_row, whose
+// quantizer takes the lanes' steps once per 4 elements ([5000, 4096] RMSNorm ->
+// Q8 19.7 us against 21.6, with the add 44.2 against 45.6).  The LDS array is
+// declared 16-byte aligned:
 // with the element type's 4-byte alignment the compiler splits every float4
 // access into two 8-byte ones.  The chains read their elements one register
 // set ahead (16 elements; 8 in the fused-add form, which keeps the weights
@@ -486,8 +498,10 @@ __global__ __launch_bounds__(TPB ? TPB : 1024) void norm_q8_row16_kernel(int8_t 
 static constexpr int row_waves(int kmax, bool add, bool few) { return few ? 1 : (kmax == 8 && add ? 4 : 8); }
 
 template <int TPR, int KMAX, bool ADD, bool LEFT, bool FEW>
-__global__ __launch_bounds__(TPR, row_waves(KMAX, ADD, FEW)) void rmsnorm_row_kernel(float *o, float *x, const float *add,
-                                                                       const float *weight, int dim, float eps) {
+__global__ __launch_bounds__(TPR, row_waves(KMAX, ADD, FEW)) void rmsnorm_row_kernel(float *o, float *x,
+                                                                                     const float *add,
+                                                                                     const float *weight, int dim,
+                                                                                     float eps) {
   rms_row<TPR, KMAX, ADD, 0, LEFT, FEW>(o, nullptr, nullptr, x, add, weight, dim, eps);
 }
 
@@ -498,17 +512,19 @@ __global__ __launch_bounds__(TPR, FEW ? 1 : 8) void rmsnorm_q8_row_kernel(int8_t
   rms_row<TPR, KMAX, ADD, QGS, false, FEW>(nullptr, q, q_s, x, add, weight, dim, eps);
 }
 
-// Many rows of exactly 4*TPR*KMAX floats with TPR = 256 (1024, 2048, 3072 and
-// 4096): the row staged at the padded layout with one 16-byte LDS store per
-// chunk, which costs the other rows on the CU less than rms_row's four 4-byte
-// ones; their waves hide the longer chain.  [8192, 4096] add+RMSNorm: 86.3 us
-// against rms_row's 89.2; [2048, 2048] 13.1 against 12.7, [512, 2048] 3.95
-// against 4.35.
-template <int KMAX, bool ADD>
-__global__ __launch_bounds__(256) void rmsnorm_fixed_row_kernel(float *o, float *xin, const float *add,
-                                                                const float *weight, int dim, float eps) {
-  constexpr int TPR = 256;
-  dim = 4 * TPR * KMAX;
+// Many rows, staged at the padded layout with one 16-byte LDS store per chunk,
+// which costs the other rows on the CU less than rms_row's four 4-byte ones and
+// its zeros; their waves hide the longer chain.  FIX: dim == 4*TPR*KMAX, every
+// chunk live (1024, 2048, 3072 and 4096 at 256 threads; with the add the weights
+// are requested ahead of the residual's stores).  Otherwise any dim up to
+// 4*TPR*KMAX, each chunk tested against the row's end and the weights read behind
+// the scale; LEFT: dim % 32 != 0.  launch_row says which rows take it.
+template <int TPR, int KMAX, bool ADD, bool FIX, bool LEFT>
+__global__ __launch_bounds__(TPR, 1) void rmsnorm_padded_row_kernel(float *o, float *xin, const float *add,
+                                                                 const float *weight, int dim, float eps) {
+  static_assert(!(FIX && LEFT), "4*TPR*KMAX is a multiple of 32");
+  constexpr bool EARLY_W = FIX && ADD;
+  if constexpr (FIX) dim = 4 * TPR * KMAX;
   extern __shared__ __attribute__((aligned(16))) float row[];
   const int tid = threadIdx.x;
   const size_t r = blockIdx.x;
@@ -517,26 +533,33 @@ __global__ __launch_bounds__(256) void rmsnorm_fixed_row_kernel(float *o, float 
 #pragma unroll
   for (int k = 0; k < KMAX; ++k) {
     const int i = 4 * (tid + k * TPR);
-    x[k] = ld_stream4(xr + i);
-    if constexpr (ADD) b[k] = ld_stream4(add + r * (size_t)dim + i);
+    if (FIX || i < dim) {
+      x[k] = ld_stream4(xr + i);
+      if constexpr (ADD) b[k] = ld_stream4(add + r * (size_t)dim + i);
+    }
   }
-  if constexpr (ADD) {
+  if constexpr (EARLY_W) {
 #pragma unroll
     for (int k = 0; k < KMAX; ++k) w[k] = *reinterpret_cast<const float4 *>(weight + 4 * (tid + k * TPR));
   }
 #pragma unroll
   for (int k = 0; k < KMAX; ++k) {
     const int i = 4 * (tid + k * TPR);
-    if constexpr (ADD) {
-      x[k] = make_float4(x[k].x + b[k].x, x[k].y + b[k].y, x[k].z + b[k].z, x[k].w + b[k].w);
-      st_stream4(xr + i, x[k]);
+    if (FIX || i < dim) {
+      if constexpr (ADD) {
+        x[k] = make_float4(x[k].x + b[k].x, x[k].y + b[k].y, x[k].z + b[k].z, x[k].w + b[k].w);
+        st_stream4(xr + i, x[k]);
+        // With a single live chunk the compiler rewrites this store into an ordinary one unless it is
+        // pinned here ([513, 1024] 3.16 us, as an ordinary store 3.46).
+        if constexpr (FIX && KMAX == 1) asm volatile("" ::: "memory");
+      }
+      *reinterpret_cast<float4 *>(row + padded(tid + k * TPR)) = x[k];
     }
-    *reinterpret_cast<float4 *>(row + padded(tid + k * TPR)) = x[k];
   }
   __syncthreads();
   // floats 16..19 of the padded layout are padding: the scale goes there
   if (tid < 64) {
-    const float s0 = rms_scale(padded_row_sumsq<8, true>(row, dim), (float)dim, eps);
+    const float s0 = rms_scale(padded_row_sumsq<8, false, LEFT>(row, dim), (float)dim, eps);
     if (tid == 0) row[16] = s0;
   }
   __syncthreads();
@@ -544,16 +567,25 @@ __global__ __launch_bounds__(256) void rmsnorm_fixed_row_kernel(float *o, float 
 #pragma unroll
   for (int k = 0; k < KMAX; ++k) {
     const int i = 4 * (tid + k * TPR);
-    if constexpr (!ADD) w[k] = *reinterpret_cast<const float4 *>(weight + i);
-    st_stream4(o + r * (size_t)dim + i, make_float4((s * x[k].x) * w[k].x, (s * x[k].y) * w[k].y,
-                                                    (s * x[k].z) * w[k].z, (s * x[k].w) * w[k].w));
+    if (FIX || i < dim) {
+      if constexpr (!EARLY_W) w[k] = *reinterpret_cast<const float4 *>(weight + i);
+      st_stream4(o + r * (size_t)dim + i, make_float4((s * x[k].x) * w[k].x, (s * x[k].y) * w[k].y,
+                                                      (s * x[k].z) * w[k].z, (s * x[k].w) * w[k].w));
+    }
   }
+}
+
+// LDS bytes of the padded layout: up to the last chunk, and at least the scale's place.
+static unsigned padded_bytes(int dim) {
+  const int m = dim / 4 - 1, end = 4 * (m + (m >> 2)) + 4, last_pad = dim % 16 ? end : dim + dim / 4;
+  return 4u * (unsigned)(last_pad < 20 ? 20 : last_pad);
 }
 
 // Calls go(tpr, kmax) with the shape as compile-time constants: kmax chunks per
 // thread, the fewest whole waves that hold dim floats.  False, and no call,
 // where that leaves more than the last chunk partly past the row's end
-// (rms_row tests only the last one) or no kernel of that size is built.
+// (rms_row tests only the last one) or the waves are outside [MIN_WAVES,
+// MAX_WAVES], the ones built.
 template <int KMAX, int MIN_WAVES, int MAX_WAVES, typename Go>
 static bool with_threads(int dim, Go go) {
   const int waves = (dim / 4 + 64 * KMAX - 1) / (64 * KMAX);
@@ -601,74 +633,177 @@ static void by_rows(int rows, int tpr, Launch launch) {
 // At most one row per CU: what counts is a row's own latency.
 constexpr int kFewRows = 256;
 
-// The row's shape, each line from the times of [rows, dim] on one MI355X:
-//  - at most 256 rows: one chunk per thread up to 1024 floats, two up to 8192,
-//    four beyond and at 4096 and 8192 (fewer waves to gather at the barriers:
-//    [8, 4096] 3.03 us against 3.22 with two);
-//  - 1024, 2048, 3072, 4096: rmsnorm_fixed_row_kernel;
-//  - above 2048 rows, below 1024 floats: a wave per row, so that more rows are
-//    resident ([3500, 896] RMSNorm 5.2 us against 6.8 with four waves; with
-//    the add the wave's registers hold only up to 768);
-//  - one chunk per thread up to 1024 floats (2048 with the add, or up to four
-//    rows per CU: [1000, 1984] RMSNorm 4.0 us against 4.3);
-//  - two chunks up to 8192, four beyond (two rows of 1024 threads per CU);
-//  - eight chunks where fewer threads per row measured faster: with the add at
-//    up to two rows per CU ([500, 5376] 8.9 us against 9.8 with two chunks),
-//    without it at two to four ([1000, 5376] 7.7 against 10.6).
+template <int N>
+using Int = std::integral_constant<int, N>;
+
+// The row's shape.  Each line follows the times of [rows, dim] on one MI355X (cold
+// rows, launches from a graph; in brackets the form it is preferred to).
+//
+// dim % 32 == 0, at most 256 rows: chains, one chunk per thread up to 1024
+// floats, two up to 8192, four beyond and at 4096 and 8192 (fewer waves to gather
+// at the barriers: [8, 4096] 3.03 us against 3.22 with two).
+//
+// More rows: chains where a row still waits mostly for itself, the padded layout,
+// whose rows cost the CU less LDS and fewer instructions, where a CU's rows wait for
+// each other:
+//  - 1024, 2048, 3072 and 4096 floats: the fixed length (so 256 without the add:
+//    its one chunk per thread needs no test);
+//  - below 1024 with the add: chains with the few-row registers up to six rows per
+//    CU ([1300, 832] 4.6 us [many-row registers 4.9]), then padded, 256 threads up to
+//    eight rows per CU ([1700, 640] 4.5 [4.8]), a wave per row ([2500, 896] 7.4 [8.5],
+//    [5000, 544] 8.5 [9.4]) until 8192 one-wave rows fill the GPU, chains beyond;
+//    without it chains, and a padded wave per row above 5000 rows ([8192, 640] 7.5
+//    [8.7]; 320 and 480 floats: at 6145 to 8191 rows);
+//  - below 2048: one chunk per thread, without the add two from four rows per CU on;
+//    with it padded, 256 threads, while a round of rows is more than 4 MB and at most
+//    eight share a CU ([1500, 1984] 9.4 [10.3], [1500, 1792] 8.4 [9.5], [769, 1152] 4.0
+//    [4.3]);
+//  - below 4096: two chunks; padded, 256 threads of four, where that makes all rows
+//    resident at once: at two to eight rows per CU with the add (six above 3072
+//    floats, [1000, 2304] 7.7 [8.4]), four to eight without ([1500, 4032] 8.2 [10.8],
+//    2560 and less from five on); three chunks and the few-row registers with
+//    the add at up to two rows per CU ([400, 2304] 4.1 [5.0]);
+//  - below 8192: two chunks; padded, 256 threads of eight, where that makes all rows
+//    resident, with the add at 449 to 1024 rows and, up to 5376 floats, again in the
+//    last part of the second round ([1000, 5376] 15.8 [17.1], [1280, 4288] 15.9 [17.6]),
+//    without it up to the rows whose LDS fits ([1300, 5376] 9.9 [12.3], [1000, 4864]
+//    7.7 [9.7]); eight chunks of chains below those where the width allows it;
+//  - beyond: four chunks; with the add up to two rows per CU padded, 256 threads of
+//    16 ([400, 12288] 16.2 [17.7]; at 8192 and 16384 eight chunks of chains), and
+//    above three rows per CU and 12288 floats the few-row registers ([1000, 14336] 42.8
+//    [46.8]; 2% slower at 16384); eight chunks at two to three rows per CU where
+//    two rows of 1024 threads leave a third waiting ([700, 10112] RMSNorm 9.9 [13.8],
+//    with the add 21.2 [23.2]).
+//
+// dim % 32 != 0 (add only; no model has such a width): padded, with half the
+// threads where that makes all rows resident ([1000, 5000] 16.0 us [17.1 with natural
+// layout, 18.9 with chains], [1500, 1032] 6.5 [8.5 with 512 threads and chains]);
+// chains from 136 to 1024 floats at up to six rows per CU ([600, 904] 3.7 [4.3]),
+// at 2056 to 8184 and above 14336 at up to one row per CU ([1, 16376] 8.8 [10.5]).
 template <bool ADD>
 static bool launch_row(float *o, float *x, const float *add, const float *weight, int rows, int dim, float eps,
                        hipStream_t stream) {
-  using std::integral_constant;
-  auto go = [&](auto tpr, auto kmax, auto leftover, auto few) {
-    constexpr int TPR = decltype(tpr)::value, K = decltype(kmax)::value;
-    constexpr bool LEFT = decltype(leftover)::value, FEW = decltype(few)::value;
-    by_rows(rows, TPR, [&](int first, int n) {
+  auto launch = [&](auto kernel, int tpr, unsigned lds) {
+    by_rows(rows, tpr, [&](int first, int n) {
       const size_t at = (size_t)first * (size_t)dim;
-      enqueue(rmsnorm_row_kernel<TPR, K, ADD, LEFT, FEW>, dim3(n), dim3(TPR),
-              ChainLayout<TPR, K, LEFT, row_chain_u(K, FEW)>::kBytes, stream, o + at, x + at, ADD ? add + at : add,
-              weight, dim, eps);
+      enqueue(kernel, dim3(n), dim3(tpr), lds, stream, o + at, x + at, ADD ? add + at : add, weight, dim, eps);
     });
     return true;
   };
-  if (dim % 32) {
-    auto left = [&](auto tpr, auto kmax) { return go(tpr, kmax, std::true_type{}, std::false_type{}); };
-    if (dim <= 256) return left(integral_constant<int, 64>{}, integral_constant<int, 1>{});
-    if (dim <= 1024) return left(integral_constant<int, 256>{}, integral_constant<int, 1>{});
-    if (dim <= 4096) return left(integral_constant<int, 512>{}, integral_constant<int, 2>{});
-    if (dim <= 8192) return left(integral_constant<int, 1024>{}, integral_constant<int, 2>{});
-    return left(integral_constant<int, 1024>{}, integral_constant<int, 4>{});
+  auto chains = [&](auto tpr, auto kmax, auto leftover, auto regs) {
+    constexpr int TPR = decltype(tpr)::value, K = decltype(kmax)::value;
+    constexpr bool LEFT = decltype(leftover)::value, FEW = decltype(regs)::value;
+    return launch(rmsnorm_row_kernel<TPR, K, ADD, LEFT, FEW>, TPR,
+                  ChainLayout<TPR, K, LEFT, row_chain_u(K, FEW)>::kBytes);
+  };
+  auto padded_rows = [&](auto tpr, auto kmax, auto leftover) {
+    constexpr int TPR = decltype(tpr)::value, K = decltype(kmax)::value;
+    return launch(rmsnorm_padded_row_kernel<TPR, K, ADD, false, decltype(leftover)::value>, TPR, padded_bytes(dim));
+  };
+  constexpr std::true_type yes{};
+  constexpr std::false_type no{};
+  if constexpr (ADD) {
+    if (dim % 32) {
+      auto pad = [&](auto tpr, auto kmax) { return padded_rows(tpr, kmax, yes); };
+      auto left = [&](auto tpr, auto kmax) { return chains(tpr, kmax, yes, no); };
+      if (dim <= 256) return dim <= 128 || rows == 1 ? pad(Int<64>{}, Int<1>{}) : left(Int<64>{}, Int<1>{});
+      if (dim <= 1024) {
+        if (rows <= 6 * kFewRows ? rows > 1 || dim > 704 : rows > 6144 && dim > 512) return left(Int<256>{}, Int<1>{});
+        if (rows <= 2048) return pad(Int<256>{}, Int<1>{});
+        return dim <= 512 ? pad(Int<64>{}, Int<2>{}) : pad(Int<64>{}, Int<4>{});
+      }
+      if (dim <= 2048) return rows <= 4 * kFewRows ? pad(Int<512>{}, Int<1>{}) : pad(Int<256>{}, Int<2>{});
+      const bool half = rows > 2 * kFewRows && rows <= 8 * kFewRows;
+      if (dim <= 4096) {
+        if (rows <= kFewRows) return left(Int<512>{}, Int<2>{});
+        return half ? pad(Int<256>{}, Int<4>{}) : pad(Int<512>{}, Int<2>{});
+      }
+      if (dim <= 8192) {
+        if (rows <= kFewRows) return left(Int<1024>{}, Int<2>{});
+        return half ? pad(Int<256>{}, Int<8>{}) : pad(Int<512>{}, Int<4>{});
+      }
+      if (rows <= kFewRows && dim > 14336) return left(Int<1024>{}, Int<4>{});
+      return rows > 384 && rows <= 576 ? pad(Int<256>{}, Int<16>{}) : pad(Int<1024>{}, Int<4>{});
+    }
   }
-  auto few = [&](auto tpr, auto kmax) { return go(tpr, kmax, std::false_type{}, std::true_type{}); };
-  auto many = [&](auto tpr, auto kmax) { return go(tpr, kmax, std::false_type{}, std::false_type{}); };
+  auto few = [&](auto tpr, auto kmax) { return chains(tpr, kmax, no, yes); };
+  auto many = [&](auto tpr, auto kmax) { return chains(tpr, kmax, no, no); };
+  auto pad = [&](auto tpr, auto kmax) { return padded_rows(tpr, kmax, no); };
   if (rows <= kFewRows) {
     if (dim <= 1024) return with_threads<1, 1, 4>(dim, few);
-    if (dim % 4096 && dim <= 8192) return with_threads<2, 3, 16>(dim, few);
-    return with_threads<4, 4, 16>(dim, few);
+    if (dim == 4096) return few(Int<256>{}, Int<4>{});
+    if (dim == 8192) return few(Int<512>{}, Int<4>{});
+    return dim < 8192 ? with_threads<2, 3, 16>(dim, few) : with_threads<4, 9, 16>(dim, few);
   }
-  auto fixed = [&](auto kmax) {
-    by_rows(rows, 256, [&](int first, int n) {
-      const size_t at = (size_t)first * (size_t)dim;
-      enqueue(rmsnorm_fixed_row_kernel<decltype(kmax)::value, ADD>, dim3(n), dim3(256),
-              (unsigned)(dim + dim / 4) * 4u, stream, o + at, x + at, ADD ? add + at : add, weight, dim, eps);
-    });
-    return true;
+  auto fixed = [&](auto tpr, auto kmax) {
+    constexpr int TPR = decltype(tpr)::value;
+    return launch(rmsnorm_padded_row_kernel<TPR, decltype(kmax)::value, ADD, true, false>, TPR, padded_bytes(dim));
   };
+  if constexpr (ADD) {
+    if (dim <= 1024 && rows <= 6 * kFewRows) return with_threads<1, 1, 4>(dim, few);
+  } else {
+    if (dim == 256) return fixed(Int<64>{}, Int<1>{});
+  }
   switch (dim) {
-    case 1024: return fixed(integral_constant<int, 1>{});
-    case 2048: return fixed(integral_constant<int, 2>{});
-    case 3072: return fixed(integral_constant<int, 3>{});
-    case 4096: return fixed(integral_constant<int, 4>{});
+    case 1024: return fixed(Int<256>{}, Int<1>{});
+    case 2048: return fixed(Int<256>{}, Int<2>{});
+    case 3072: return fixed(Int<256>{}, Int<3>{});
+    case 4096: return fixed(Int<256>{}, Int<4>{});
   }
-  const bool two_per_cu = rows <= 2 * kFewRows, four_per_cu = rows <= 4 * kFewRows;
-  if (rows > 2048 && dim > 256 && dim <= (ADD ? 768 : 1024)) {
-    if (dim <= 512) return many(integral_constant<int, 64>{}, integral_constant<int, 2>{});
-    if (dim <= 768) return many(integral_constant<int, 64>{}, integral_constant<int, 3>{});
-    return many(integral_constant<int, 64>{}, integral_constant<int, 4>{});
+  if (dim < 1024) {
+    if constexpr (ADD)
+      if (dim > 512 && rows <= 2048) return pad(Int<256>{}, Int<1>{});
+    if (dim > 512 && (ADD ? rows < 8192 : rows > 5000)) return pad(Int<64>{}, Int<4>{});
+    if (rows > 2048 && dim > 256) {
+      if constexpr (!ADD)
+        if (dim <= 512 && rows > 6144 && rows < 8192) return pad(Int<64>{}, Int<2>{});
+      if (dim <= 512) return many(Int<64>{}, Int<2>{});
+      if (dim <= 768) return many(Int<64>{}, Int<3>{});
+      if constexpr (!ADD) return many(Int<64>{}, Int<4>{});
+    }
+    if constexpr (ADD)
+      return dim <= 512 ? with_threads<1, 1, 2>(dim, many) : many(Int<256>{}, Int<1>{});
+    else
+      return with_threads<1, 1, 4>(dim, many);
   }
-  if (dim <= 1024 || (dim <= 2048 && (ADD || four_per_cu))) return with_threads<1, 1, 8>(dim, many);
-  if (dim <= 4096) return with_threads<2, 3, 8>(dim, many);
-  if ((ADD ? two_per_cu : four_per_cu && !two_per_cu && dim < 8192) && with_threads<8, 3, 8>(dim, many)) return true;
-  return dim < 8192 ? with_threads<2, 9, 16>(dim, many) : with_threads<4, 8, 16>(dim, many);
+  if (dim < 2048) {
+    if constexpr (ADD)
+      return rows > 2 * kFewRows && rows <= 8 * kFewRows && rows * dim > 1 << 20 ? pad(Int<256>{}, Int<2>{})
+                                                                                 : with_threads<1, 5, 8>(dim, many);
+    else
+      return rows <= 4 * kFewRows ? with_threads<1, 5, 8>(dim, many) : with_threads<2, 3, 4>(dim, many);
+  }
+  if (dim < 4096) {
+    if (rows > (ADD ? 2 : dim <= 2560 ? 5 : 4) * kFewRows && rows <= (ADD && dim > 3072 ? 6 : 8) * kFewRows)
+      return pad(Int<256>{}, Int<4>{});
+    if constexpr (ADD)
+      if (rows <= 2 * kFewRows && dim <= 3840) return with_threads<3, 3, 6>(dim, few);
+    return with_threads<2, 5, 8>(dim, many);
+  }
+  if (dim < 8192) {
+    // rows of the padded layout that are resident at once: 5 bytes of LDS a float, 68 VGPRs (seven workgroups)
+    const int on_cu = 160 * 1024 / (5 * dim), resident = kFewRows * (on_cu < 7 ? on_cu : 7);
+    if (ADD ? (rows > 448 && rows <= 4 * kFewRows) ||
+                  (dim < 5632 && rows > 1152 && rows <= (dim <= 5120 ? 1536 : 1280))
+            : rows <= resident && rows > (dim <= 4608 ? 3 : dim < 5376 ? 2 : 4) * kFewRows)
+      return pad(Int<256>{}, Int<8>{});
+    if ((ADD ? rows <= 448 : rows > 2 * kFewRows && rows <= 4 * kFewRows) && with_threads<8, 3, 4>(dim, many))
+      return true;
+    return with_threads<2, 9, 16>(dim, many);
+  }
+  if constexpr (ADD) {
+    if (rows <= 2 * kFewRows) {
+      if (dim == 8192) return many(Int<256>{}, Int<8>{});
+      if (dim == 16384) return many(Int<512>{}, Int<8>{});
+      return pad(Int<256>{}, Int<16>{});
+    }
+    if (rows <= 3 * kFewRows && dim > 8192 && dim <= 10240 && with_threads<8, 5, 5>(dim, many)) return true;
+    if (rows > 3 * kFewRows && dim > 12288 && dim < 16384) return with_threads<4, 13, 16>(dim, few);
+  } else {
+    if (rows > 2 * kFewRows && rows <= 3 * kFewRows && dim > 9216 && dim < 12288 && with_threads<8, 5, 6>(dim, many))
+      return true;
+  }
+  return with_threads<4, 8, 16>(dim, many);
 }
 
 bool launch_fused_add_rmsnorm(float *o, float *residual, const float *add, const float *weight, int rows, int dim,
@@ -680,12 +815,19 @@ bool launch_rmsnorm(float *o, const float *x, const float *weight, int rows, int
   return launch_row<false>(o, const_cast<float *>(x), nullptr, weight, rows, dim, eps, stream);
 }
 
+// RMSNorm -> Q8 as one row of chains: at most 256 rows, and more where
+// norm_q8_row16_kernel cannot (below 512 or above 12288 floats, codes off their
+// 16-byte boundary).  More rows, from [rows, dim] with unaligned codes: with the add
+// one chunk per thread up to 4096 floats, four with the few-row registers up to 8192
+// and above 12288 ([512, 8192] 11.5 us [two chunks 12.6]); without it one chunk while few
+// rows share a CU, then two up to 2048 and four beyond ([2048, 3840] 9.3 us [one
+// chunk 12.3], [1000, 8192] 9.9 [two 15.3]).
 template <int QGS, bool ADD>
 static bool launch_q8_row(int8_t *q, float *q_s, float *x, const float *add, const float *weight, int rows, int dim,
                           float eps, hipStream_t stream) {
-  auto go = [&](auto tpr, auto kmax, auto few) {
+  auto go = [&](auto tpr, auto kmax, auto regs) {
     constexpr int TPR = decltype(tpr)::value, K = decltype(kmax)::value;
-    constexpr bool FEW = decltype(few)::value;
+    constexpr bool FEW = decltype(regs)::value;
     by_rows(rows, TPR, [&](int first, int n) {
       const size_t at = (size_t)first * (size_t)dim;
       enqueue(rmsnorm_q8_row_kernel<TPR, K, QGS, ADD, FEW>, dim3(n), dim3(TPR),
@@ -696,11 +838,25 @@ static bool launch_q8_row(int8_t *q, float *q_s, float *x, const float *add, con
   };
   auto few = [&](auto tpr, auto kmax) { return go(tpr, kmax, std::true_type{}); };
   auto many = [&](auto tpr, auto kmax) { return go(tpr, kmax, std::false_type{}); };
-  if (rows > 2048 && dim > 256 && dim <= 512)
-    return many(std::integral_constant<int, 64>{}, std::integral_constant<int, 2>{});
-  if (dim <= 4096) return with_threads<1, 1, 16>(dim, few);
-  if (dim <= 8192) return with_threads<2, 9, 16>(dim, few);
-  return rows <= kFewRows ? with_threads<4, 9, 16>(dim, few) : with_threads<4, 9, 16>(dim, many);
+  if (rows > 2048 && dim > 256 && dim <= 512) return many(Int<64>{}, Int<2>{});
+  if (dim <= 4096) {
+    if constexpr (!ADD) {
+      if (dim > 1024 && dim <= 2048 && rows > 4 * kFewRows) return with_threads<2, 3, 4>(dim, many);
+      if (dim > 2048 && rows > 2 * kFewRows)
+        return with_threads<4, 3, 4>(dim, many) || with_threads<2, 5, 5>(dim, many);
+    }
+    return with_threads<1, 1, 16>(dim, few);
+  }
+  if (dim <= 8192) {
+    if (rows <= (ADD ? 1 : 2) * kFewRows) return with_threads<2, 9, 16>(dim, few);
+    if constexpr (ADD)
+      return dim <= 5632 ? with_threads<2, 9, 11>(dim, few) : with_threads<4, 6, 8>(dim, few);
+    else
+      return with_threads<4, 5, 8>(dim, many);
+  }
+  const bool few_regs = dim == 16384 || (dim > 12288 && rows > 3 * kFewRows) || (dim < 12288 && QGS == 32);
+  if (rows <= kFewRows || (ADD && few_regs)) return with_threads<4, 9, 16>(dim, few);
+  return with_threads<4, ADD && QGS == 32 ? 12 : 9, 16>(dim, many);
 }
 
 bool launch_rmsnorm_quantize(int8_t *q, float *q_s, float *x, const float *add, const float *weight, int rows,

@@ -1,8 +1,8 @@
 // row_dispatch.hip -- the launches that the row kernels' dispatch makes, without a GPU.
 //
 // Compiled for the host only and linked without the HIP runtime: enqueue() is
-// replaced by a recorder, so every accepted shape of the three row entries can be
-// asked for its launches.  For each shape the recorded
+// replaced by a recorder, so every accepted shape of the three row entries and of
+// the quantizer can be asked for its launches.  For each shape the recorded
 // launches must together cover every row once, in order, each with fewer than 2^32
 // threads and at most 160 KiB of LDS, by a kernel whose threads and chunks hold the
 // row.  Prints one line per fault, then the names of all kernels chosen.
@@ -35,6 +35,7 @@ static void record(void (*kernel)(K...), dim3 grid, dim3 block, unsigned lds, hi
 
 #define enqueue record
 #include "../v7multiplikator_amd/csrc/k_add_rmsnorm.hip"
+#include "../v7multiplikator_amd/csrc/k_swiglu_q8.hip"
 #undef enqueue
 
 // The registration hooks of the host object; nothing is registered or launched.
@@ -139,6 +140,23 @@ int main() {
         }
       }
     }
+  // The quantizer: fewer than 2^32 threads for every accepted size.
+  const float *in = reinterpret_cast<const float *>(kBase);
+  int8_t *q = reinterpret_cast<int8_t *>(kBase * 2);
+  for (int gs : {1, 3, 16, 32, 64, 100, 128, 256, 512, 4096})
+    for (long long len : {1ll, 64ll, 4096ll, 12288ll, 16385ll, 1ll << 20, 1ll << 30})
+      for (long long n : {1ll << 20, (1ll << 34) - 4096, 1ll << 34, (1ll << 34) + (1ll << 20), 1ll << 36, (1ll << 40) - 1}) {
+        const long long r = n / len;
+        if (r < 1 || r > 2147483647 || r * ((len + gs - 1) / gs) >= 1ll << 38) continue;
+        for (int off : {0, 1}) {
+          launches.clear();
+          v7g::launch_quantize_q8(q + off, qs, in, nullptr, nullptr, (int)r, (int)len, gs, nullptr);
+          if (launches.size() != 1) fault("quantizer launches", "quantize", r, len, gs, "");
+          for (const Launch &l : launches)
+            if ((unsigned long long)l.grid.x * l.block.x >= 1ull << 32)
+              fault("grid of 2^32 threads", "quantize", r, len, gs, name_of(l.kernel).c_str());
+        }
+      }
   for (const std::string &n : names) std::printf("KERNEL %s\n", n.c_str());
   std::printf("%d faults\n", faults);
   return faults != 0;

@@ -67,6 +67,7 @@ def test_more_lanes_than_32_bits_index(ops):
     """2^31 lanes (a group of 1 per lane) and more take 64-bit indices: the same codes and scales as calls over
     parts of the array, around the 2^31 element boundary and at both ends."""
     rows, row_len = (1 << 31) // 100 + 9, 100
+    torch.cuda.empty_cache()
     free, _ = torch.cuda.mem_get_info()
     if free < 40 << 30:
         pytest.skip("needs 40 GB of free device memory")
@@ -78,3 +79,33 @@ def test_more_lanes_than_32_bits_index(ops):
     for r0 in (0, at - 8, rows - 16):
         pq, ps = ops.quantize_q8(x[r0:r0 + 16].contiguous(), gs=1)
         assert torch.equal(q[r0:r0 + 16], pq) and torch.equal(s[r0:r0 + 16], ps)
+
+
+@pytest.mark.parametrize("gs,row_len,rows", [
+    (64, 65, (1 << 26) + 9),   # 16 lanes a group, every second group of one element
+    (32, 33, (1 << 27) + 9),   # 8 lanes a group
+    (257, 258, (1 << 24) + 9),  # 64 lanes a group that walk it in steps, every second group of one element
+    (64, 64, (1 << 28) + 9),   # whole groups, one lane per 4 elements would be 2^32 lanes
+])
+def test_64_bit_lane_indices_with_partial_groups(ops, gs, row_len, rows):
+    """2^31 lanes and more with a 64-bit division of the group index by the groups of a row: the same codes and scales
+    as calls over a few rows, at both ends and on both sides of the 2^31st lane and the 2^32nd element."""
+    n = rows * row_len
+    torch.cuda.empty_cache()
+    free, _ = torch.cuda.mem_get_info()
+    if free < 7 * n:
+        pytest.skip("needs 7 bytes of free device memory per element")
+    x = torch.rand(rows, row_len, device="cuda")
+    spr = -(-row_len // gs)
+    lanes = 64 if gs > 256 else gs // 4
+    starts = sorted({0, rows - 16, *(min(max(at - 8, 0), rows - 16) for at in ((1 << 31) // (spr * lanes),
+                                                                               (1 << 32) // row_len))})
+    for r0 in starts:
+        x[r0, row_len - 1] = float("nan")
+        x[r0 + 9, 3] = float("inf")
+        x[r0 + 10, row_len - 1] = 5.0
+    q, s = ops.quantize_q8(x, gs=gs)
+    s = s.view(rows, spr)
+    for r0 in starts:
+        pq, ps = ops.quantize_q8(x[r0:r0 + 16].contiguous(), gs=gs)
+        assert torch.equal(q[r0:r0 + 16], pq) and torch.equal(s[r0:r0 + 16], ps.view(16, spr)), r0

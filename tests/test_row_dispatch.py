@@ -1,6 +1,6 @@
-"""The dispatch of the row kernels over every accepted width and extreme row counts, on the CPU (row_dispatch.hip):
-each call launches something, every row is covered once, no grid reaches HIP's limit of 2^32 threads, and every row
-kernel that is built can be chosen."""
+"""The dispatch of the row kernels and the quantizer over every accepted width and extreme row counts, on the CPU
+(row_dispatch.hip): each call launches something, every row is covered once, no grid reaches HIP's limit of 2^32
+threads, and every row kernel that is built can be chosen."""
 from __future__ import annotations
 
 import os

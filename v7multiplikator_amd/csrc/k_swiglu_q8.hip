@@ -316,9 +316,8 @@ static bool aligned(const void *p, size_t a) { return p == nullptr || ((uintptr_
 void launch_quantize_q8(int8_t *out_q, float *out_s, const float *x, const float *gate, const float *up, int rows,
                         int row_len, int gs, hipStream_t stream) {
   const long long n = (long long)rows * row_len;
-  // one lane per 4 elements in a 32-bit grid; beyond it the group kernel (32 and 64: the launch is refused)
-  const bool flat_grid = gs == 32 || gs == 64 || n / 4 < (1LL << 32) - 256;
-  const bool flat = row_len % gs == 0 && flat_grid && aligned(out_q, 4) && aligned(x, 16) &&
+  // one lane per 4 elements, fewer than 2^32 (HIP's limit of a grid); beyond it the group kernel's grid-stride loop
+  const bool flat = row_len % gs == 0 && n / 4 < (1LL << 32) - 256 && aligned(out_q, 4) && aligned(x, 16) &&
                     aligned(gate, 16) && aligned(up, 16);
   if (flat) {
     auto go = [&](auto g) { launch_flat<decltype(g)::value>(out_q, out_s, x, gate, up, n, stream); };

@@ -235,6 +235,10 @@ float v7g_get_rms_eps(void);
 int v7g_get_last_error(void);
 void v7g_clear_last_error(void);
 const char *v7g_error_string(int code);
+/* The tag of this header that the library was built with (a digest of its
+ * text): a binding compiled on its own, which calls the entries by address,
+ * compares it with the tag that it was built with. */
+const char *v7g_header_tag(void);
 /* Library-owned RoPE tables built by v7s_rope_init / v7g_rope_init. */
 int v7g_get_rope_tables(float **cos_table, float **sin_table, int *rope_max_dim, int *n_pos);
 /* As v7s_rope_init with an explicit position count (1 .. 131072). */

@@ -42,6 +42,7 @@ SIGNATURES = {
     "v7g_get_last_error": (_i, []),
     "v7g_clear_last_error": (None, []),
     "v7g_error_string": (ctypes.c_char_p, [_i]),
+    "v7g_header_tag": (ctypes.c_char_p, []),
     "v7g_get_rope_tables": (_i, [_vp, _vp, _vp, _vp]),
     "v7g_rope_init": (_i, [_i, _f, _i]),
     "v7g_build_rope_tables": (_i, [_vp, _vp, _i, _i, _f]),

@@ -12,6 +12,7 @@ packed-FP32 instructions disabled (-Xclang -target-feature -Xclang
 from __future__ import annotations
 
 import glob
+import hashlib
 import os
 import shutil
 import subprocess
@@ -34,6 +35,16 @@ HIP_FLAGS = [
     "-mllvm", "-amdgpu-kernarg-preload-count=14",
     "-Wall", "-Wno-unused-function",
 ]
+
+
+HEADER = os.path.join(ROOT, "include", "v7g_lib.h")
+
+
+def header_tag_flag() -> str:
+    """The define that tells the library and the separately compiled _ops_native which v7g_lib.h they were built
+    with."""
+    with open(HEADER, "rb") as f:
+        return f'-DV7G_HEADER_TAG="{hashlib.sha256(f.read()).hexdigest()[:16]}"'
 
 
 def hipcc() -> str:
@@ -72,7 +83,7 @@ def build_library(verbose: bool = False) -> str:
             raise RuntimeError(f"g++ failed ({res.returncode}):\n{res.stdout}{res.stderr}")
         objs.append(obj)
     exports = os.path.join(CSRC, "v7g_exports.map")
-    cmd = [hipcc(), *HIP_FLAGS, "-I", os.path.join(ROOT, "include"), f"-Wl,--version-script={exports}", "-o", tmp,
+    cmd = [hipcc(), *HIP_FLAGS, header_tag_flag(), "-I", os.path.join(ROOT, "include"), f"-Wl,--version-script={exports}", "-o", tmp,
            *sources(), "-x", "none", *objs]
     if verbose:
         print(" ".join(cmd), flush=True)
@@ -96,11 +107,14 @@ def build_native(verbose: bool = False) -> str:
     import torch
     from torch.utils import cpp_extension
 
+    from .ops import torch_build
+
     src = os.path.join(PKG, "native", "ops_native.cpp")
     out = os.path.join(PKG, "_ops_native.so")
     lib_dirs = [os.path.join(os.path.dirname(torch.__file__), "lib")]
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           header_tag_flag(), f'-DV7G_TORCH_BUILD="{torch_build()}"',
            *[a for p in cpp_extension.include_paths() for a in ("-isystem", p)],
            "-isystem", sysconfig.get_paths()["include"], "-o", out + ".tmp", src,
            *[f"-L{d}" for d in lib_dirs], "-lc10", "-ltorch_cpu", "-ltorch_python"]

@@ -335,6 +335,11 @@ const char *v7g_error_string(int code) {
   }
 }
 
+#ifndef V7G_HEADER_TAG
+#define V7G_HEADER_TAG "untagged"  // built without build.py: no separately compiled binding matches
+#endif
+const char *v7g_header_tag(void) { return V7G_HEADER_TAG; }
+
 int v7g_build_rope_tables(float *cos_table, float *sin_table, int n_pos, int head_dim, float rope_base) {
   if (!cos_table || !sin_table) return fail(V7G_ERR_NULL);
   if (int rc = check_table_shape(n_pos, head_dim)) return fail(rc);

@@ -590,4 +590,17 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_ops_native", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__ops_native(void) { return PyModule_Create(&module); }
+#if !defined(V7G_HEADER_TAG) || !defined(V7G_TORCH_BUILD)
+#error "build.py defines V7G_HEADER_TAG and V7G_TORCH_BUILD"
+#endif
+
+// ops uses the module only where both attributes match the library and the torch that are running.
+PyMODINIT_FUNC PyInit__ops_native(void) {
+  PyObject *m = PyModule_Create(&module);
+  if (m && (PyModule_AddStringConstant(m, "header_tag", V7G_HEADER_TAG) < 0 ||
+            PyModule_AddStringConstant(m, "torch_build", V7G_TORCH_BUILD) < 0)) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

@@ -29,6 +29,7 @@ from __future__ import annotations
 import ctypes
 import importlib.util
 import os
+import sys
 
 import torch
 
@@ -78,13 +79,21 @@ class _Unbound:
         global _fast
         try:
             L = _lib.load()
-        except RuntimeError:  # the Python body meets it again, after its own checks
+        except (RuntimeError, OSError, AttributeError):  # the Python body meets it again, after its own checks
             return lambda *args: None
         _fast = _bind_native(L)
         return getattr(_fast, name)
 
 
+def torch_build() -> str:
+    """Which torch and Python: the module reads tensors through the headers of the one that it was built against."""
+    return (f"{torch.__version__} {torch.version.git_version} "
+            f"{sys.implementation.name}-{sys.version_info[0]}.{sys.version_info[1]}")
+
+
 def _bind_native(L):
+    """The module, or no native path where it is not there, does not load, or was built for another torch or Python
+    or with another include/v7g_lib.h than L: neither tensors nor the library may then be read through it."""
     device = getattr(torch._C, "_cuda_getDevice", None)
     if _raw_stream is None or device is None or not os.path.exists(_NATIVE_PATH):
         return _NoNative()
@@ -92,7 +101,10 @@ def _bind_native(L):
     try:
         mod = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(mod)
-    except ImportError:  # built against another torch
+    except ImportError:  # a symbol that this torch does not have
+        return _NoNative()
+    if (getattr(mod, "torch_build", None), getattr(mod, "header_tag", None)) != (torch_build(),
+                                                                                 L.v7g_header_tag().decode()):
         return _NoNative()
     mod.bind({n: ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in _lib.SIGNATURES}, _raw_stream, device,
              _lib.check)

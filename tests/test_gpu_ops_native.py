@@ -55,6 +55,10 @@ def calls():
             got = o.fused_add_rmsnorm(r, rnd(3, 5, 64, seed=1), w.detach() if given else w, eps=1e-5, out=buf)
             return got, r, buf, got is buf
 
+        def one_row(o, given=given):  # a contiguous row whose first stride is no row length
+            r = rnd(9, 64).as_strided((1, 64), (99, 1))
+            return o.fused_add_rmsnorm(r, rnd(1, 64), rnd(64)), o.rmsnorm(r, rnd(64)), o.swiglu(r, r)
+
         def norm(o, given=given):
             x = rnd(5, 96)
             buf = x if given else None
@@ -103,7 +107,7 @@ def calls():
             buf = torch.zeros(6, 32, dtype=torch.float16, device="cuda") if given else None
             return o.kv_pack_f16_kv(src[:, :32], src[:, 32:], v_out=buf)
 
-        for f in (fused, norm, nq8, anq8, sw, swq, quant, emb, pack, pack2):
+        for f in (fused, one_row, norm, nq8, anq8, sw, swq, quant, emb, pack, pack2):
             add(f"{f.__name__}-{tag}", f)
 
         def heads(o, given=given):

@@ -167,7 +167,8 @@ struct Rows {
 };
 
 at::Tensor out_like(const Call &c, int i, const at::Tensor &like) {
-  if (c.none(i)) return at::empty(like.sizes(), like.options().requires_grad(false));
+  // contiguous, with like's own strides where a dimension of one element leaves them free, as torch.empty_like
+  if (c.none(i)) return at::empty_strided(like.sizes(), like.strides(), like.options().requires_grad(false));
   const at::Tensor &o = c.f(i);
   need(o.sizes() == like.sizes());
   return o;

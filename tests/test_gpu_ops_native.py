@@ -211,3 +211,42 @@ def test_follows_the_current_stream(ops):
     ops.add_inplace(x, x.clone())
     assert (_lib.load().v7g_get_stream() or 0) == torch.cuda.current_stream().cuda_stream
     torch.cuda.synchronize()
+
+
+# With an allocator that counts: every op that allocates its results, through the native path.
+UNDER_THE_GIL = """
+import ctypes, sys
+import torch
+path = sys.argv[1]
+torch.cuda.memory.change_current_allocator(torch.cuda.memory.CUDAPluggableAllocator(path, "gil_alloc", "gil_free"))
+from v7multiplikator_amd import _lib, ops
+count = ctypes.PyDLL(path)
+x, w = torch.ones(8, 64, device="cuda"), torch.ones(64, device="cuda")
+ids = torch.zeros(3, dtype=torch.int32, device="cuda")
+tq, ts = torch.ones(5, 64, device="cuda").to(torch.int8), torch.ones(5, device="cuda")
+ops.add_inplace(x, x.clone())
+assert ops._fast.__name__ == "_ops_native"
+held, made = count.gil_held(), count.gil_all()
+keep = [ops._fast.fused_add_rmsnorm(x, x.clone(), w, 1e-6, None), ops._fast.rmsnorm(x, w, 1e-6, None),
+        ops._fast.rmsnorm_quantize(x, w, 1e-6, 64, None, None),
+        ops._fast.add_rmsnorm_quantize(x, x.clone(), w, 1e-6, 64, None, None), ops._fast.swiglu(x, x, None),
+        ops._fast.swiglu_q8(x, x, 64, None, None), ops._fast.quantize_q8(x, 64, None, None),
+        ops._fast.embedding_gather_q8(ids, tq, ts, None), ops._fast.kv_pack_f16(x, None),
+        ops._fast.kv_pack_f16_kv(x, x, None, None)]
+assert all(k is not None for k in keep)
+torch.cuda.synchronize()
+print("HELD", count.gil_held() - held, "OF", count.gil_all() - made)
+"""
+
+
+def test_results_are_allocated_without_the_gil():
+    """An allocation may reach the driver; torch.empty lets the other threads run meanwhile, and so do the ops."""
+    import os
+    import subprocess
+    import sys
+
+    here = os.path.dirname(os.path.abspath(__file__))
+    res = subprocess.run([sys.executable, "-c", UNDER_THE_GIL, os.path.join(here, "libgil_alloc.so")],
+                         capture_output=True, text=True, timeout=100, cwd=os.path.dirname(here))
+    assert res.returncode == 0, res.stderr
+    assert "HELD 0 OF 17" in res.stdout, res.stdout

@@ -171,6 +171,22 @@ def build_test_shim(verbose: bool = False) -> str:
     return out
 
 
+def build_gil_alloc(verbose: bool = False) -> str:
+    """Test support: tests/libgil_alloc.so, a torch allocator that counts allocations made under the GIL."""
+    import sysconfig
+
+    src = os.path.join(ROOT, "tests", "gil_alloc.c")
+    out = os.path.join(ROOT, "tests", "libgil_alloc.so")
+    cmd = ["gcc", "-O2", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+           "-I", sysconfig.get_paths()["include"], "-o", out, src, "-L/opt/rocm/lib", "-lamdhip64"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"gcc failed ({res.returncode}):\n{res.stdout}{res.stderr}")
+    return out
+
+
 if __name__ == "__main__":
     print(build_library(verbose=True))
     print(build_native(verbose=True))

@@ -129,15 +129,16 @@ struct Call {
   }
 };
 
-// Releases the GIL, as ctypes does around a call (a launch may wait for room in the queue).
+// Releases the GIL, as ctypes does around a call (a launch may wait for room in the queue) and torch.empty around
+// an allocation (which may reach the driver).
 struct NoGil {
   PyThreadState *state = PyEval_SaveThread();
   ~NoGil() { PyEval_RestoreThread(state); }
 };
 
 template <typename F>
-int without_gil(F call) {
-  NoGil g;
+auto without_gil(F call) {
+  const NoGil g;
   return call();
 }
 
@@ -168,7 +169,9 @@ struct Rows {
 
 at::Tensor out_like(const Call &c, int i, const at::Tensor &like) {
   // contiguous, with like's own strides where a dimension of one element leaves them free, as torch.empty_like
-  if (c.none(i)) return at::empty_strided(like.sizes(), like.strides(), like.options().requires_grad(false));
+  if (c.none(i))
+    return without_gil(
+        [&] { return at::empty_strided(like.sizes(), like.strides(), like.options().requires_grad(false)); });
   const at::Tensor &o = c.f(i);
   need(o.sizes() == like.sizes());
   return o;
@@ -180,18 +183,19 @@ struct Q8Out {
 Q8Out q8_out(const Call &c, int iq, int is, const at::Tensor &like, const Rows &r, int gs) {
   const int64_t spr = (static_cast<int64_t>(r.dim) + gs - 1) / gs;
   Q8Out o;
-  const auto opt = at::TensorOptions().device(like.device());
-  if (c.none(iq)) {
-    o.q = at::empty(like.sizes(), opt.dtype(at::kChar));
-  } else {
+  if (!c.none(iq)) {
     o.q = c.t(iq, at::kChar);
     need(o.q.numel() == static_cast<int64_t>(r.rows) * r.dim);
   }
-  if (c.none(is)) {
-    o.s = at::empty({static_cast<int64_t>(r.rows), spr}, opt.dtype(at::kFloat));
-  } else {
+  if (!c.none(is)) {
     o.s = c.t(is, at::kFloat);
     need(o.s.numel() == r.rows * spr);
+  }
+  if (!o.q.defined() || !o.s.defined()) {
+    const NoGil g;
+    const auto opt = at::TensorOptions().device(like.device());
+    if (!o.q.defined()) o.q = at::empty(like.sizes(), opt.dtype(at::kChar));
+    if (!o.s.defined()) o.s = at::empty({static_cast<int64_t>(r.rows), spr}, opt.dtype(at::kFloat));
   }
   return o;
 }
@@ -367,7 +371,9 @@ PyObject *embedding_gather_q8(const Call &c) {  // ids, table_q, table_s, out
   need(ts.numel() == static_cast<int64_t>(vocab) * dim / 64);
   at::Tensor o;
   if (c.none(3)) {
-    o = at::empty({static_cast<int64_t>(n), static_cast<int64_t>(dim)}, ts.options().requires_grad(false));
+    o = without_gil([&] {
+      return at::empty({static_cast<int64_t>(n), static_cast<int64_t>(dim)}, ts.options().requires_grad(false));
+    });
   } else {
     o = c.f(3);
     need(o.numel() == static_cast<int64_t>(n) * dim);
@@ -481,7 +487,9 @@ const at::Tensor &rows_view(const Call &c, int i, at::ScalarType type) {
   return t;
 }
 at::Tensor f16_out(const Call &c, int i, const at::Tensor &src) {
-  if (c.none(i)) return at::empty(src.sizes(), at::TensorOptions().device(src.device()).dtype(at::kHalf));
+  if (c.none(i))
+    return without_gil(
+        [&] { return at::empty(src.sizes(), at::TensorOptions().device(src.device()).dtype(at::kHalf)); });
   const at::Tensor &o = c.t(i, at::kHalf, false);
   need(o.sizes() == src.sizes() && o.stride(1) == 1);
   return o;

@@ -194,6 +194,67 @@ def test_native_is_the_python_path(ops, monkeypatch, f):
             assert a == b
 
 
+class Recorder:
+    """Stands in for the native module and notes what each call answered: True where it made the call (a library error
+    counts: the library was asked), False where it declined."""
+
+    def __init__(self, mod):
+        self.mod, self.made = mod, []
+
+    def __getattr__(self, name):
+        def call(*args):
+            try:
+                r = getattr(self.mod, name)(*args)
+            except Exception:
+                self.made.append(True)
+                raise
+            self.made.append(r is not None)
+            return r
+        return call
+
+
+# What is not the plain accepted call: declined, or (qk with a K cache) never asked.
+DECLINED = {"qk-given": [], "zero_dim": [False], "zero_width": [False], "transposed": [False], "double": [False],
+            "host": [False], "not_a_tensor": [False], "shape": [False], "weight_size": [False], "gs_zero": [False],
+            "gs_negative": [False], "gs_float": [False], "eps_text": [False], "out_size": [False],
+            "positions": [False], "heads_dim": [False], "heads_apart": [False], "pos0_large": [False],
+            "keep_int": [False], "table_scales": [False], "subclass": [False]}
+CALLS_PER_FORM = {"one_row": 3, "heads": 2}
+
+
+@pytest.mark.parametrize("name,f", [pytest.param(p.id, p.values[0], id=p.id) for p in calls()])
+def test_native_makes_the_accepted_calls(ops, monkeypatch, name, f):
+    """Which forms the native path serves itself: falling through to Python gives the same results, so only this
+    shows an entry that has stopped accepting."""
+    rec = Recorder(ops._fast)
+    monkeypatch.setattr(ops, "_fast", rec)
+    outcome(f, ops)
+    assert rec.made == DECLINED.get(name, [True] * CALLS_PER_FORM.get(name.split("-")[0], 1))
+
+
+def test_native_declines_under_torch_modes(ops, monkeypatch):
+    """A torch function or dispatch mode must see the Python path's torch calls."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x, w = rnd(4, 64), rnd(64)
+    want = ops.rmsnorm(x, w)
+    for mode in (Function, Dispatch):
+        rec = Recorder(ops._fast)
+        with monkeypatch.context() as m, mode():
+            m.setattr(ops, "_fast", rec)
+            got = ops.rmsnorm(x, w)
+        assert rec.made == [False] and torch.equal(got, want)
+
+
 def test_follows_the_current_stream(ops):
     """Work queued on a side stream is seen by a native call made under that stream, and by no other."""
     from v7multiplikator_amd import _lib

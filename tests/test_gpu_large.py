@@ -190,7 +190,7 @@ def test_embedding_gather_on_both_sides_of_the_32_bit_dword_limit(ops):
 
 
 def test_quantize_q8_generic_rows_past_2_pow_32_elements(ops, oracle):
-    """Q8 quantize (GS 64) of rows of 4100 floats (the general kernel: one thread per group, a 4-element tail
+    """Q8 quantize (GS 64) of rows of 4100 floats (the group kernel: 16 lanes per group, a 4-element tail
     group per row) over 1,047,553 rows = 4,294,967,300 elements; sampled rows against the oracle."""
     rows, row_len = 1047553, 4100
     need(4 * rows * row_len + rows * row_len + rows * 65 * 4)

@@ -122,11 +122,8 @@ def test_fused_add_rmsnorm_validator_shapes(ops, oracle, dim, seed):
         assert_bits(host(got_o), want_o, "o")
 
 
-# Model widths: each compiled-in shape of the fixed-length row (2560, 3072, 3584, 3840, 5120, 8192), the run-time
-# thread count with 1, 2 and 4 chunks per thread (1280, 1536 / 6144, 7168 / none below 8192 beyond those), the
-# dispatch shapes (2048, 4096) and a multiple of 256 that falls back to the general kernel (4352); below 1024, the
-# 256-thread row at the padded layout and, where the width is not a multiple of 32 (520, 776, 1000), at the natural
-# one (more than 2048 such rows take one wave each: test_one_wave_rows).
+# Model widths at few rows: chains of one, two and four chunks per thread on 1 to 16 waves, and rows that end in
+# leftover 8-float blocks (520, 776, 1000).  More rows take other kernels: test_gpu_row_shapes.py.
 MODEL_WIDTHS = [264, 320, 384, 512, 520, 576, 640, 768, 776, 896, 960, 1000,
                 1280, 1536, 2048, 2560, 3072, 3584, 3840, 4096, 4352, 5120, 6144, 7168, 8192]
 
@@ -149,9 +146,9 @@ def test_fused_add_rmsnorm_model_widths(ops, oracle, dim):
 
 @pytest.mark.parametrize("dim", [264, 320, 448, 512, 520, 576, 640, 768, 776, 896, 960, 1000])
 def test_one_wave_rows(ops, oracle, dim):
-    """More than 2048 rows below 1024 floats: one wave per row with 2, 3 or 4 float4 chunks per lane, full (512,
-    768) and partial, at the padded layout and the natural one (520, 776, 1000), through add+RMSNorm, RMSNorm,
-    RMSNorm -> Q8 and its fused-add form (below 512: the 16-elements-per-thread quantizer starts at 512)."""
+    """More than 2048 rows below 1024 floats: one wave per row (padded with the add above 512 floats and for rows that
+    end in leftover 8-float blocks, as chains otherwise), through add+RMSNorm, RMSNorm, RMSNorm -> Q8 and its
+    fused-add form (from 512 floats on the 16-elements-per-thread quantizer)."""
     rows = 2309
     r = C.normal(dim + 5, (rows, dim))
     a = C.normal(dim + 6, (rows, dim))
@@ -550,8 +547,8 @@ def test_rmsnorm_quantize_nan_columns(ops, oracle, gs):
 @pytest.mark.parametrize("dim", [544, 4096, 12288])
 def test_rmsnorm_quantize_nan_at_every_group_position(ops, oracle, gs, dim):
     """A NaN weight at each position of a quantization group in turn (group g: position g % gs), beside a
-    weight of 2^20 two positions on, through the 16-elements-per-thread kernel (dims 544: a partial wave of
-    34 threads, GS 32 only; 4096; 12288): the reference's ordered vmaxps tree keeps the NaN or drops it with
+    weight of 2^20 two positions on, at a few rows (the row kernel's 4 elements per lane; test_gpu_row16.py has
+    the 16-elements-per-thread kernel): the reference's ordered vmaxps tree keeps the NaN or drops it with
     its partners (src/asm/rmsnorm_quantize_kernel.inc:158-187).  Also with the residual add fused in front."""
     if dim % gs:
         pytest.skip("dim must be a multiple of the group size")
@@ -666,10 +663,10 @@ def test_add_rmsnorm_quantize_equals_the_two_calls(ops, oracle, gs, dim):
 @pytest.mark.parametrize("rows,dim", [(64, 4096), (2309, 768)])
 @pytest.mark.parametrize("fused_add", [False, True])
 def test_rmsnorm_quantize_codes_4_byte_aligned(ops, oracle, gs, rows, dim, fused_add):
-    """Codes that are 4-byte but not 16-byte aligned (the C ABI accepts them) send dims 512..12288 to the row
-    kernel's 4-elements-per-lane quantizer instead of the 16-per-thread kernel: [64, 4096] runs the 256-thread
-    row, [2309, 768] (more than 2048 rows) the one-wave row.  Through the C ABI, plain and with the fused add,
-    bit-exact against the oracle; the bytes around the codes stay untouched."""
+    """Codes that are 4-byte but not 16-byte aligned (the C ABI accepts them) send more than 256 rows of 512..12288
+    floats to the row kernel's 4-elements-per-lane quantizer instead of the 16-per-thread kernel ([2309, 768]);
+    [64, 4096] takes the row kernel either way.  Through the C ABI, plain and with the fused add, bit-exact
+    against the oracle; the bytes around the codes stay untouched."""
     import ctypes
 
     from v7multiplikator_amd import _lib
@@ -1182,7 +1179,8 @@ def denormal_mix(seed, shape):
 def test_denormal_rows_norms_follow_ftz_daz(ops, oracle, eps, dim):
     """add+RMSNorm, RMSNorm, RMSNorm->Q8 and the fused add->RMSNorm->Q8 on rows of denormals and tiny values,
     bit for bit with the oracle in the reference's MXCSR FTZ+DAZ mode (eps = 0 lets an all-flushed sum of
-    squares give an infinite scale).  dim 4096 takes the 16-elements-per-thread RMSNorm->Q8 kernel."""
+    squares give an infinite scale).  16 rows: the row kernels; test_gpu_row16.py has the 16-elements-per-thread
+    RMSNorm->Q8 kernel."""
     r = denormal_mix(501, (16, dim))
     a = denormal_mix(502, (16, dim))[::-1].copy()
     w = C.norm_weight(503, dim)

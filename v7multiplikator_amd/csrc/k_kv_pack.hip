@@ -43,10 +43,11 @@ __global__ __launch_bounds__(256) void kv_pack_f16_kernel(uint16_t *dst, long lo
 // token's K and V stretch of the QKV row side by side.  Measured at 8192
 // tokens x 1024: 17.7 us against 18.6 us for one thread per chunk of either
 // side and 20.6-21.1 us for two launches.  Strides below 2^32 elements go as
-// 32-bit arguments (S = unsigned): the arguments then fill 13 dwords, all of
-// which the firmware preloads into SGPRs at wave launch, where with 64-bit
-// strides the chunk count and the row count come past the 14 preloaded
-// dwords and each wave waits for a scalar load of them first.
+// 32-bit arguments (S = unsigned): the arguments that the row-per-workgroup form
+// reads then fill 13 dwords, all of which the firmware preloads into SGPRs at
+// wave launch, where with 64-bit strides the chunk count and the row count come
+// past the 14 preloaded dwords and each wave waits for a scalar load of them
+// first.  The flat form's reciprocal lies past them in either case.
 template <typename S, bool FLAT>
 __global__ __launch_bounds__(256) void kv_pack2_f16_kernel(uint16_t *k_dst, uint16_t *v_dst, const float *k_src,
                                                            const float *v_src, S k_dst_stride, S v_dst_stride,

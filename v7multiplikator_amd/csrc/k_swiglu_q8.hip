@@ -10,14 +10,15 @@
 //     tail group uses the same arithmetic.
 //   The SwiGLU -> Q8 chain (src/asm/prefill_q8.inc:1154-1183) quantizes the
 //   SwiGLU row; here the SwiGLU values never leave registers.
-// The reference group size is 64 (src/asm/v7_core.inc:120); GS is a template
-// parameter so 32-element blocks use the same algorithm.
+// The reference group size is 64 (src/asm/v7_core.inc:120); 32-element blocks
+// and the other group sizes use the same algorithm.
 //
 // Vector layout: lane owns 4 consecutive floats (streaming dwordx4 loads of
-// gate and up, or x), GS/4 consecutive lanes form one group, the group max is
-// a DPP butterfly inside 8 or 16 lanes (the reference's ordered vmaxps tree in
-// a wave that holds a NaN or an Inf), each lane stores its 4 codes as one
-// dword, and the first lane of the group stores the scale.  The divisions of
+// gate and up, or x), a power of two of consecutive lanes (1 to 64) forms one
+// group, the group max is a lane butterfly inside them (for full groups of 32
+// and 64 the reference's ordered vmaxps tree in a wave that holds a NaN or an
+// Inf), each lane stores its 4 codes as one dword, and the first lane of the
+// group stores the scale.  The divisions of
 // the reference (sigmoid's 1/(1+e), wmax/127, 1/scale) are the shorter
 // sequences of v7g_device.h that give the same bits for every reachable input.
 #include <type_traits>

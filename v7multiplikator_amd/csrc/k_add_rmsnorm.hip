@@ -817,9 +817,10 @@ bool launch_rmsnorm(float *o, const float *x, const float *weight, int rows, int
 
 // RMSNorm -> Q8 as one row of chains: at most 256 rows, and more where
 // norm_q8_row16_kernel cannot (below 512 or above 12288 floats, codes off their
-// 16-byte boundary).  More rows, from [rows, dim] with unaligned codes: with the add
-// one chunk per thread up to 4096 floats, four with the few-row registers up to 8192
-// and above 12288 ([512, 8192] 11.5 us [two chunks 12.6]); without it one chunk while few
+// 16-byte boundary).  More rows, from [rows, dim] with unaligned codes: one chunk
+// per thread keeps the few-row registers at any row count ([100000, 256] 28.9 us
+// [many-row registers 31.8], [20000, 1024] 23.2 [25.5]); with the add one chunk per
+// thread up to 4096 floats, four with the few-row registers up to 8192 and above 12288 ([512, 8192] 11.5 us [two chunks 12.6]); without it one chunk while few
 // rows share a CU, then two up to 2048 and four beyond ([2048, 3840] 9.3 us [one
 // chunk 12.3], [1000, 8192] 9.9 [two 15.3]).
 template <int QGS, bool ADD>

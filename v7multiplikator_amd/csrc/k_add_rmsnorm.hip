@@ -817,12 +817,16 @@ bool launch_rmsnorm(float *o, const float *x, const float *weight, int rows, int
 
 // RMSNorm -> Q8 as one row of chains: at most 256 rows, and more where
 // norm_q8_row16_kernel cannot (below 512 or above 12288 floats, codes off their
-// 16-byte boundary).  More rows, from [rows, dim] with unaligned codes: one chunk
-// per thread keeps the few-row registers at any row count ([100000, 256] 28.9 us
-// [many-row registers 31.8], [20000, 1024] 23.2 [25.5]); with the add one chunk per
-// thread up to 4096 floats, four with the few-row registers up to 8192 and above 12288 ([512, 8192] 11.5 us [two chunks 12.6]); without it one chunk while few
-// rows share a CU, then two up to 2048 and four beyond ([2048, 3840] 9.3 us [one
-// chunk 12.3], [1000, 8192] 9.9 [two 15.3]).
+// 16-byte boundary).  More rows, from [rows, dim] with unaligned codes (in brackets
+// the shape that the line is preferred to):
+//  - one chunk per thread, up to 4096 floats with the add and while few rows share a
+//    CU without it, keeps the few-row registers at any row count ([100000, 256]
+//    28.9 us [many-row registers 31.8], [20000, 1024] 23.2 [25.5]);
+//  - without the add then two chunks up to 2048 floats and four beyond, many-row
+//    registers ([2048, 3840] 9.8 [one chunk 13.0], [1000, 8192] 9.9 [two 15.3]);
+//  - with the add two chunks up to 5632 floats, four beyond, with the few-row
+//    registers up to 8192 ([5000, 8192] 91 [two chunks 104]), at 16384 ([400, 16384]
+//    21.7 [24.1]), above 12288 from three rows per CU on and below it at GS 32.
 template <int QGS, bool ADD>
 static bool launch_q8_row(int8_t *q, float *q_s, float *x, const float *add, const float *weight, int rows, int dim,
                           float eps, hipStream_t stream) {
